@@ -61,7 +61,7 @@ ROWS = {
     "K12 find_ntuplets": (("startMask", "startCompact", "ntupletCount", "ntupletScan", "ntupletFill"),
                           lambda c: 8 * c["C"] + 4 * c["L"] + 14 * c["T"]),
     "K13 cleaners/multiplicity/classify": (("trackListAlloc", "trackListFill", "trackListSort", "multiplicity",
-                                            "classify", "dupPreds", "fastDuplicate", "hitToTupleCount",
+                                            "classify", "dupActive", "fastDuplicate", "hitToTupleCount",
                                             "hitToTupleScan", "hitToTupleFill", "tripletCleaner"),
                                            lambda c: 8 * c["C"] + 300 * c["T"]),
     "K14 broken-line fits": (("fit",), lambda c: 22 * c["Nbar"] * c["T"] + 92 * c["T"]),
@@ -82,7 +82,7 @@ KERNEL_LABEL = {
     "trackListFillKernel": "trackListFill", "trackListBuildKernel": "trackListFill",
     "trackListSortKernel": "trackListSort",
     "multiplicityKernel": "multiplicity", "fitKernel": "fit", "classifyKernel": "classify",
-    "dupPredsKernel": "dupPreds", "fastDuplicateKernel": "fastDuplicate", "hitToTupleCountKernel": "hitToTupleCount",
+    "dupActiveKernel": "dupActive", "fastDuplicateKernel": "fastDuplicate", "hitToTupleCountKernel": "hitToTupleCount",
     "hitToTupleScanKernel": "hitToTupleScan", "hitToTupleFillKernel": "hitToTupleFill",
     "hitToTupleBuildKernel": "hitToTupleFill",
     "tripletCleanerKernel": "tripletCleaner", "vertexKernel": "vertices",

@@ -134,7 +134,7 @@ typedef struct {
   uint32_t *hitToTupleOff; uint32_t* hitToTupleBins;
   uint32_t counts[20];   /* nCells, nDoublets, apcM, apcN, nTuples, status, nbLists, trLists,
                             nMulti, nMult, nVertices, vtxTracks, vstatus, nSlots, nNeighbors, nStart,
-                            nPaths, 0, 0, 0 */
+                            nPaths, nActive, 0, 0 */
 } pxg_ca_internals;
 
 /* Context: device + conditions uploaded once, immutable afterwards (pxg_init is the

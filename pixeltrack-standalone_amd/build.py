@@ -3,7 +3,7 @@
   libpxgen.so   synthetic event source (g++)
   libpxhost.so  host FED loop and the EDM-style framework with its plugins (g++)
   libpxgpu.so   HIP kernels + C ABI (hipcc --offload-arch=gfx950)
-  tests/native/libpxprim_selftest.so   self-test kernels of the device primitives (tests only)
+  tests/native/libpx*_selftest.so   self-test kernels of single device parts (tests only)
 
 Every call compiles (no staleness check): the build is the "does it build" check.
 """
@@ -53,10 +53,11 @@ def build_gpu():
 
 
 def build_selftest():
-    """Self-test kernels of the shared device primitives (tests/native), for the GPU tests."""
-    src = os.path.join(REPO, "tests", "native", "primitives_selftest.hip")
-    if os.path.exists(src):
-        _run([HIPCC] + HIP_FLAGS + [src, "-o", os.path.join(REPO, "tests", "native", "libpxprim_selftest.so")])
+    """Self-test kernels (tests/native), for the GPU tests."""
+    for name, lib in (("primitives", "prim"), ("duplicates", "duplicates")):
+        src = os.path.join(REPO, "tests", "native", f"{name}_selftest.hip")
+        if os.path.exists(src):
+            _run([HIPCC] + HIP_FLAGS + [src, "-o", os.path.join(REPO, "tests", "native", f"libpx{lib}_selftest.so")])
 
 
 def build_framework():

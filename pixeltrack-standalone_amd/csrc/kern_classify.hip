@@ -4,9 +4,9 @@
 //
 // The serial fast duplicate remover visits cells in index order and each
 // visit depends on the qualities left by earlier visits of cells that share a
-// tuple.  Here a cell is processed once every lower-index cell sharing one of
-// its tuples has been processed (rounds inside one workgroup per event);
-// cells that share no tuple commute, so the result is the serial one.  The
+// tuple.  Here the cells with two or more loose tuples are visited in rounds
+// inside one workgroup per event, each once every lower one sharing a loose
+// tuple has been; cells that share none commute, so the result is the serial one.  The
 // triplet cleaner and the hit -> tuple fill only mark duplicates from
 // quantities that do not change meanwhile, so they run per hit in parallel.
 #include <hip/hip_runtime.h>
@@ -28,6 +28,7 @@ namespace pxg {
       const uint32_t* off = ca.tupleOff + ca.offBase(e);
       const float c0 = float(0.68177776), c1 = float(0.74609577), c2 = float(-0.08035491), c3 = float(0.00315399);
       for (uint32_t t = gridStart(); t < nT; t += gridStride()) {
+        ca.dupOwner[tb + t] = 0xffffffffu;  // for the duplicate remover
         const uint32_t nh = off[t + 1] - off[t];
         // the serial loop stops at the first empty tuple; only the last stored
         // tuple can be empty (when the container overflowed)
@@ -72,207 +73,222 @@ namespace pxg {
       }
     }
 
-    // a21 kernel_fastDuplicateRemover.  The serial loop visits the cells with two
-    // or more tuples in ascending order, keeps the loose tuple with the smallest
-    // |tip| of each and marks the other (not bad) tuples duplicates.  A cell's
-    // outcome depends only on the lower cells sharing one of its tuples (its
-    // predecessors), so cells run in rounds: a cell is processed once all its
-    // predecessors have been, and the cells of one round share no tuple.
+    // a21 kernel_fastDuplicateRemover.  The serial loop visits the cells with two or more
+    // tuples in ascending order, keeps the loose tuple with the smallest |tip| of each and
+    // marks its other tuples that are not bad duplicates.  A visit therefore changes
+    // something only if two or more of the cell's tuples are loose, and loose tuples only
+    // ever become duplicates: a cell with fewer than two loose tuples when the remover
+    // starts is left out for good.  That leaves 1k of 5k cells at PU50 and 17k of 44k at
+    // PU200, with two loose tuples each on average.
+    //
+    // dupActiveKernel (the whole grid) lists those cells with their loose tuples and |tip|,
+    // plane by plane so that the rounds below read them coalesced; the rounds run in one
+    // workgroup per event.
 
-    // the predecessors of cell c: lower cells with two or more tuples in its tuples
-    template <typename F>
-    __device__ __forceinline__ void forPreds(const CAPool& ca, size_t cb, size_t tb, const TupleIndex* pool, uint32_t c,
-                                             F&& f) {
-      const TupleIndex* list = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
-      const uint32_t n = ca.trCount[cb + c];
-      for (uint32_t a = 0; a < n; ++a) {
-        const uint32_t* cells = ca.tupleCells + 4 * tb + 4 * size_t(list[a]);
-        for (int k2 = 0; k2 < 4; ++k2) {
-          const uint32_t o = cells[k2];
-          if (o == 0xffffffffu)
-            break;
-          if (o < c && ca.trCount[cb + o] >= 2 && f(o))
-            return;
-        }
-      }
-    }
+    constexpr uint32_t kDupOver = 255;  // more loose tuples than kept: read from the track list
 
-    // keep the loose tuple of cell c with the smallest |tip|, the others are duplicates
-    __device__ __forceinline__ void dupProcess(const CAPool& ca, size_t cb, const TupleIndex* pool, uint8_t* q,
-                                               const float* tip, uint32_t c) {
-      const TupleIndex* list = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
-      const uint32_t n = ca.trCount[cb + c];
-      float mc = 10000.f;
-      TupleIndex im = kNoTuple;
-      for (uint32_t a = 0; a < n; ++a) {
-        const TupleIndex it = list[a];
-        const float score = fabsf(tip[it]);
-        if (q[it] == kQualityLoose && score < mc) {
-          mc = score;
-          im = it;
-        }
-      }
-      for (uint32_t a = 0; a < n; ++a) {
-        const TupleIndex it = list[a];
-        if (q[it] != kQualityBad && it != im)
-          q[it] = kQualityDup;
-      }
-    }
-
-    // the first kDupPredCap predecessors of every cell with two or more tuples
-    // (all slots written, unused ones ~0), on the whole grid
-    __global__ void __launch_bounds__(kCaBlock) dupPredsKernel(CAPool ca) {
+    __global__ void __launch_bounds__(kCaBlock) dupActiveKernel(CAPool ca) {
       const uint32_t e = logicalBlock().y;
       const uint32_t nMulti = ca.cnt[e].nMulti;
       const size_t cb = ca.cellBase(e);
       const size_t tb = ca.tupleBase(e);
-      const size_t lb = size_t(e) * ca.caps.maxCellLists;
+      const uint32_t L = ca.caps.maxCellLists;
+      const size_t lb = size_t(e) * L;
       const uint32_t* multi = ca.multiCells + cb;
       const TupleIndex* pool = ca.trPool + lb * kCaMaxCellTracks;
-      uint32_t* preds = ca.dupPreds + lb * kDupPredCap;
-      for (uint32_t k = gridStart(); k < nMulti; k += gridStride()) {
-        uint32_t m = 0;
-        uint32_t keep[kDupPredCap];
+      const uint8_t* q = ca.quality + tb;
+      const float* tip = ca.state + 5 * tb + 1 * size_t(ca.caps.maxTuples);
+      const uint32_t lane = laneId();
+      for (uint32_t k0 = gridStart() - lane; k0 < nMulti; k0 += gridStride()) {  // uniform per wave
+        const uint32_t k = k0 + lane;
+        uint32_t c = 0, m = 0;
+        uint32_t keep[kDupLooseCap];
+        if (k < nMulti) {
+          c = multi[k];
+          const TupleIndex* list = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
+          const uint32_t n = ca.trCount[cb + c];
+          for (uint32_t a = 0; a < n; ++a) {
+            const TupleIndex it = list[a];
+            if (q[it] != kQualityLoose)
+              continue;
 #pragma unroll
-        for (uint32_t j = 0; j < kDupPredCap; ++j)
-          keep[j] = 0xffffffffu;
-        bool over = false;
-        forPreds(ca, cb, tb, pool, multi[k], [&](uint32_t o) {
-          bool seen = false;
-#pragma unroll
-          for (uint32_t j = 0; j < kDupPredCap; ++j)
-            seen |= keep[j] == o;
-          if (seen)
-            return false;
-          if (m == kDupPredCap) {
-            over = true;  // more distinct predecessors than kept: walked when needed
-            return true;
+            for (uint32_t j = 0; j < kDupLooseCap; ++j)
+              keep[j] = j == m ? it : keep[j];
+            ++m;
           }
+        }
+        const bool active = m >= 2;
+        const uint32_t at = waveAlloc(&ca.cnt[e].nActive, active);
+        if (active) {
+          ca.dupCells[lb + at] = c;
+          ca.dupCount[lb + at] = m <= kDupLooseCap ? uint8_t(m) : uint8_t(kDupOver);
+          uint2* rec = ca.dupLoose + lb * kDupLooseCap + at;
 #pragma unroll
-          for (uint32_t j = 0; j < kDupPredCap; ++j)
-            if (j == m)
-              keep[j] = o;
-          ++m;
-          return false;
-        });
+          for (uint32_t j = 0; j < kDupLooseCap; ++j)
+            if (j < m)
+              rec[size_t(j) * L] = make_uint2(keep[j], __float_as_uint(fabsf(tip[keep[j]])));
+          // the first round's owner of each tuple
+          if (m <= kDupLooseCap) {
 #pragma unroll
-        for (uint32_t j = 0; j < kDupPredCap; ++j)
-          preds[size_t(k) * kDupPredCap + j] = keep[j];
-        ca.dupCount[lb + k] = over ? uint8_t(255) : uint8_t(m);
+            for (uint32_t j = 0; j < kDupLooseCap; ++j)
+              if (j < m)
+                atomicMin(&ca.dupOwner[tb + keep[j]], c);
+          } else {
+            const TupleIndex* list = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
+            for (uint32_t a = 0; a < ca.trCount[cb + c]; ++a)
+              if (q[list[a]] == kQualityLoose)
+                atomicMin(&ca.dupOwner[tb + list[a]], c);
+          }
+        }
       }
     }
 
-    constexpr uint32_t kDupBitmapCells = kCapsReference.maxDoublets;  // done bits of the cells in LDS
+    // The listed cells of one event in rounds.  A cell may be visited once every lower
+    // listed cell that shares a tuple still loose with it has been; the cells of one round
+    // share no loose tuple, so their visits commute and the result is the serial one.
+    // Every tuple has an owner, the lowest pending cell that has it loose, and a cell that
+    // owns all its loose tuples is visited.  The first round's owners were taken on the
+    // whole grid, one per tuple; it leaves a third of the cells at PU50 and a fifth at
+    // PU200.  Those stand in an LDS list (if at most kDupList), and the later rounds take
+    // owners with an LDS atomicMin in a table of tuple indices modulo its size: two tuples
+    // on one slot only make the higher cell wait a round longer.  A cell left with fewer
+    // than two loose tuples is done at once.  The lowest pending cell is always visited, so
+    // the rounds end; 3 to 6 are taken.
+    //
+    // Bound: one CU's latency and its rate of scattered accesses.  The loose flags are
+    // therefore bits in LDS, filled by one coalesced pass over the qualities, the tuples'
+    // |tip| stands in the cells' records, and the records are read coalesced.
+    // Against rounds over all cells with two or more tuples and their predecessors: one
+    // PU50 event 75 to 11 us, 128 of them 161 to 25 us, 12 PU200 events (which went by
+    // flags in memory) 2608 to 113 us; the listing on the grid costs what finding the
+    // predecessors did (11 to 7, 83 to 59 and 65 to 62 us).
+    constexpr uint32_t kDupSlots = 16384;
+    constexpr uint32_t kDupList = 8192;
 
     __global__ void __launch_bounds__(kEventBlock) fastDuplicateKernel(CAPool ca) {
       const uint32_t e = blockIdx.x;
-      const uint32_t nMulti = ca.cnt[e].nMulti;
-      const uint32_t nCells = ca.cnt[e].nCells;
+      __shared__ uint32_t slot[kDupSlots];
+      __shared__ uint32_t loose[kCapsHighOccupancy.maxTuples / 32];  // bit t: tuple t is loose
+      __shared__ uint32_t list[2][kDupList];                          // pending cells (record indices)
+      __shared__ uint32_t nList[2];
+      static_assert(kCapsReference.maxTuples <= kCapsHighOccupancy.maxTuples && kCapsReference.maxTuples % 32 == 0,
+                    "loose bits");
+      const uint32_t n = ca.cnt[e].nActive;
+      if (n == 0)
+        return;
+      const uint32_t nT = ca.cnt[e].nTuples;
       const size_t cb = ca.cellBase(e);
       const size_t tb = ca.tupleBase(e);
-      const size_t lb = size_t(e) * ca.caps.maxCellLists;
-      const uint32_t M = ca.caps.maxTuples;
-      const uint32_t* multi = ca.multiCells + cb;
+      const uint32_t L = ca.caps.maxCellLists;
+      const size_t lb = size_t(e) * L;
       const TupleIndex* pool = ca.trPool + lb * kCaMaxCellTracks;
-      const uint32_t* preds = ca.dupPreds + lb * kDupPredCap;
-      const uint8_t* count = ca.dupCount + lb;
+      const uint32_t* cells = ca.dupCells + lb;
+      const uint2* recs = ca.dupLoose + lb * kDupLooseCap;
+      const uint32_t* owner = ca.dupOwner + tb;
+      uint8_t* count = ca.dupCount + lb;
       uint8_t* q = ca.quality + tb;
-      const float* tip = ca.state + 5 * tb + 1 * size_t(M);
+      const float* tip = ca.state + 5 * tb + 1 * size_t(ca.caps.maxTuples);
 
-      // ---- done bits of all cells in LDS; each thread keeps its (at most kDupPer)
-      // cells with their predecessors from dupPredsKernel in registers
-      constexpr uint32_t kDupPer = 6;
-      __shared__ uint32_t sDone[kDupBitmapCells / 32];
-      bool lds = nCells <= kDupBitmapCells && nMulti <= kDupPer * kEventBlock;
-      uint32_t myC[kDupPer], myN[kDupPer], myP[kDupPer][kDupPredCap];
-      if (lds) {
+      auto isLoose = [&](TupleIndex it) { return (loose[it >> 5] >> (it & 31)) & 1; };
+      // f(tuple, |tip|) on the cell's tuples that are loose now, in ascending order
+      auto forLoose = [&](uint32_t k, uint32_t m, auto&& f) {
+        if (m <= kDupLooseCap) {
+          uint2 r[kDupLooseCap];
 #pragma unroll
-        for (uint32_t i = 0; i < kDupPer; ++i) {
-          const uint32_t k = threadIdx.x + i * kEventBlock;
-          myN[i] = 0;
-          myC[i] = 0;
-          if (k < nMulti) {
-            myC[i] = multi[k];
-            myN[i] = count[k];
+          for (uint32_t j = 0; j < kDupLooseCap; ++j)
+            if (j < m)
+              r[j] = recs[size_t(j) * L + k];
 #pragma unroll
-            for (uint32_t j = 0; j < kDupPredCap; ++j)
-              myP[i][j] = preds[size_t(k) * kDupPredCap + j];
-          }
+          for (uint32_t j = 0; j < kDupLooseCap; ++j)
+            if (j < m && isLoose(r[j].x))
+              f(r[j].x, __uint_as_float(r[j].y));
+        } else {
+          const uint32_t c = cells[k];
+          const TupleIndex* tracks = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
+          const uint32_t nl = ca.trCount[cb + c];
+          for (uint32_t a = 0; a < nl; ++a)
+            if (isLoose(tracks[a]))
+              f(tracks[a], fabsf(tip[tracks[a]]));
         }
-        for (uint32_t w = threadIdx.x; w < (nCells + 31) / 32; w += kEventBlock)
-          sDone[w] = 0;
-        __syncthreads();
+      };
+
+      // sixteen qualities per thread and load (an event's stride is a multiple of sixteen)
+      uint16_t* half = reinterpret_cast<uint16_t*>(loose);
+      for (uint32_t i = threadIdx.x; i < (nT + 15) / 16; i += kEventBlock) {
+        const uint4 v = reinterpret_cast<const uint4*>(q)[i];
+        uint32_t bits = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < 16; ++b) {
+          const uint32_t w = b < 4 ? v.x : b < 8 ? v.y : b < 12 ? v.z : v.w;
+          bits |= uint32_t(((w >> (8 * (b % 4))) & 0xff) == kQualityLoose) << b;
+        }
+        half[i] = uint16_t(bits);
       }
-      if (lds) {
-        auto done = [&](uint32_t c) { return (sDone[c >> 5] >> (c & 31)) & 1; };
-        uint32_t mine = 0;  // bit i: cell i of this thread still pending
-#pragma unroll
-        for (uint32_t i = 0; i < kDupPer; ++i)
-          mine |= uint32_t(threadIdx.x + i * kEventBlock < nMulti) << i;
-        // the lowest pending cell is always ready: nMulti + 1 rounds bound the loop
-        for (uint32_t round = 0; round <= nMulti; ++round) {
-          uint32_t now = 0;  // processed in this round
-#pragma unroll
-          for (uint32_t i = 0; i < kDupPer; ++i) {
-            if (!((mine >> i) & 1))
-              continue;
-            bool ready = true;
-            if (myN[i] <= kDupPredCap) {
-#pragma unroll
-              for (uint32_t j = 0; j < kDupPredCap; ++j)
-                ready = ready && (j >= myN[i] || done(myP[i][j]));
-            } else {  // too many predecessors to keep: walk them
-              forPreds(ca, cb, tb, pool, myC[i], [&](uint32_t o) {
-                ready = done(o);
-                return !ready;
-              });
-            }
-            if (!ready)
-              continue;
-            dupProcess(ca, cb, pool, q, tip, myC[i]);
-            now |= 1u << i;
+      if (threadIdx.x < 2)
+        nList[threadIdx.x] = 0;
+      __syncthreads();
+      bool listed = false;  // the pending cells stand in list[round & 1]
+      uint32_t nPending = n;
+      for (uint32_t round = 0; round <= n; ++round) {
+        const uint32_t* pend = list[round & 1];
+        uint32_t* next = list[(round + 1) & 1];
+        if (round > 0) {
+          for (uint32_t i = threadIdx.x; i < nPending; i += kEventBlock) {
+            const uint32_t k = listed ? pend[i] : i;
+            const uint32_t m = count[k], c = cells[k];
+            if (m)
+              forLoose(k, m, [&](TupleIndex it, float) { atomicMin(&slot[it % kDupSlots], c); });
           }
           __syncthreads();
-#pragma unroll
-          for (uint32_t i = 0; i < kDupPer; ++i)
-            if ((now >> i) & 1)
-              atomicOr(&sDone[myC[i] >> 5], 1u << (myC[i] & 31));
-          mine &= ~now;
-          if (!__syncthreads_or(mine != 0))
-            break;
         }
-        return;
-      }
-
-      // ---- otherwise the same rounds over per-cell flags in memory (bit2
-      // processed, bit3 processed in this round) and the full predecessor walk
-      for (uint32_t round = 0; round <= nMulti; ++round) {
-        int pending = 0;
-        for (uint32_t k = threadIdx.x; k < nMulti; k += kEventBlock) {
-          const uint32_t c = multi[k];
-          if (ca.cellFlags[cb + c] & 4)
-            continue;
-          bool ready = true;
-          forPreds(ca, cb, tb, pool, c, [&](uint32_t o) {
-            ready = (ca.cellFlags[cb + o] & 4) != 0;
-            return !ready;
+        // The visits of this round.  A visited cell owns all of its loose tuples, so no
+        // other visit touches them; a cell that has to wait may see a tuple it does not
+        // own as loose or already as a duplicate, and waits or goes by the rest, which it
+        // owns: either is the serial order.
+        for (uint32_t i = threadIdx.x; i < nPending; i += kEventBlock) {
+          const uint32_t k = listed ? pend[i] : i;
+          const uint32_t m = count[k], c = cells[k];
+          if (m == 0)
+            continue;  // done
+          bool mine = true;
+          uint32_t alive = 0;
+          float mc = 10000.f;
+          TupleIndex im = kNoTuple;
+          forLoose(k, m, [&](TupleIndex it, float score) {
+            mine = mine && (round > 0 ? slot[it % kDupSlots] : owner[it]) == c;
+            ++alive;
+            if (score < mc) {
+              mc = score;
+              im = it;
+            }
           });
-          if (!ready) {
-            pending = 1;
-            continue;
+          if (alive >= 2) {
+            if (!mine) {
+              const uint32_t at = waveAlloc(&nList[(round + 1) & 1], true);
+              if (at < kDupList)
+                next[at] = k;
+              continue;
+            }
+            forLoose(k, m, [&](TupleIndex it, float) {
+              if (it != im) {
+                q[it] = kQualityDup;
+                atomicAnd(&loose[it >> 5], ~(1u << (it & 31)));
+              }
+            });
           }
-          dupProcess(ca, cb, pool, q, tip, c);
-          ca.cellFlags[cb + c] |= 8;  // done in this round
+          count[k] = 0;
         }
         __syncthreads();
-        for (uint32_t k = threadIdx.x; k < nMulti; k += kEventBlock) {
-          const uint32_t c = multi[k];
-          const uint8_t f = ca.cellFlags[cb + c];
-          if (f & 8)
-            ca.cellFlags[cb + c] = uint8_t((f & ~8) | 4);
-        }
-        if (!__syncthreads_or(pending))
+        const uint32_t left = nList[(round + 1) & 1];
+        if (left == 0)
           break;
+        listed = left <= kDupList;
+        nPending = listed ? left : n;
+        for (uint32_t i = threadIdx.x; i < kDupSlots; i += kEventBlock)
+          slot[i] = 0xffffffffu;
+        if (threadIdx.x == 0)
+          nList[round & 1] = 0;
+        __syncthreads();
       }
     }
 
@@ -465,8 +481,8 @@ namespace pxg {
       fishboneCleanerKernel<<<dim3(l.blocks, l.nEvents), kCaBlock, 0, l.s>>>(*l.ca);
       l.t->e();
     }
-    l.t->b("dupPreds");
-    dupPredsKernel<<<dim3(l.blocks, l.nEvents), kCaBlock, 0, l.s>>>(*l.ca);
+    l.t->b("dupActive");
+    dupActiveKernel<<<dim3(l.blocks, l.nEvents), kCaBlock, 0, l.s>>>(*l.ca);
     l.t->e();
     l.t->b("fastDuplicate");
     fastDuplicateKernel<<<l.nEvents, kEventBlock, 0, l.s>>>(*l.ca);

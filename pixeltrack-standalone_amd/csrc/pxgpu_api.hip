@@ -123,7 +123,9 @@ namespace pxg::detail {
     f(ca.trCount, D);
     f(ca.trPool, L * kCaMaxCellTracks);
     f(ca.multiCells, D);
-    f(ca.dupPreds, L * kDupPredCap);
+    f(ca.dupCells, L);
+    f(ca.dupLoose, L * kDupLooseCap);
+    f(ca.dupOwner, T);
     f(ca.dupCount, L);
     f(ca.tupleOff, E * (ca.caps.maxTuples + 64));
     f(ca.tupleBins, 5 * T);
@@ -234,7 +236,9 @@ namespace pxg::detail {
     v.trCount += D;
     v.trPool += L * kCaMaxCellTracks;
     v.multiCells += D;
-    v.dupPreds += L * kDupPredCap;
+    v.dupCells += L;
+    v.dupLoose += L * kDupLooseCap;
+    v.dupOwner += T;
     v.dupCount += L;
     v.tupleOff += c.offBase(first);
     v.tupleBins += 5 * T;

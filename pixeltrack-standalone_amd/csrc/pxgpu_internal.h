@@ -136,7 +136,7 @@ namespace pxg {
   constexpr uint32_t kListsInLdsMinEvents = 8;               // batches this large build lists per event in LDS
   // vertex clustering algorithms (gpuVertexFinder.h:46-60; density is the reference's default)
   enum : int { kVertexDensity = 0, kVertexDBSCAN = 1, kVertexIterative = 2 };
-  constexpr uint32_t kDupPredCap = 6;                        // predecessors kept per cell for the duplicate remover
+  constexpr uint32_t kDupLooseCap = 6;                       // loose tuples kept per cell for the duplicate remover
 
   // ---- XCD-aware workgroup order -------------------------------------------------------
   // The dispatcher hands workgroups to the chip's 8 XCDs round-robin by linear
@@ -180,6 +180,7 @@ namespace pxg {
     uint32_t nNeighbors;   // neighbour entries stored
     uint32_t nStart;       // cells the ntuplet walk starts from
     uint32_t nPaths;       // tuples whose path the counting walk recorded
+    uint32_t nActive;      // cells with two or more loose tuples before the duplicate remover
   };
 
   // Device arrays of the ntuplet and vertex stages, all per event at e * stride
@@ -191,7 +192,7 @@ namespace pxg {
     uint64_t* dMask;         // [2 * kDoubletSlots]: accepted candidates of a slot's first 128
     uint16_t *cellInner, *cellOuter;  // [maxDoublets]
     uint8_t* cellPair;
-    uint8_t* cellFlags;      // bit0 listed in its outer hit's list, bit1 killed, bit2 duplicate pass done
+    uint8_t* cellFlags;      // bit1 killed
     uint8_t* cellUsed;       // [maxDoublets] 1: the cell has a neighbour or is one
     uint32_t* ohCount;       // [kHitStride] cells per outer hit, then fill cursors
     uint32_t* ohOff;         // [kHitStride]
@@ -207,8 +208,10 @@ namespace pxg {
     uint16_t* trCount;       // [maxDoublets] tracks of the cell (about 20 at PU200), then stored (<= 48)
     TupleIndex* trPool;      // [maxCellLists * 48]
     uint32_t* multiCells;    // [maxDoublets] cells with two or more tracks (any order)
-    uint32_t* dupPreds;      // [maxCellLists * 8] per multiCells entry: its lower cells sharing a tuple (first 8)
-    uint8_t* dupCount;       // [maxCellLists] their number, 255 if more than 8
+    uint32_t* dupCells;      // [maxCellLists] cells with two or more loose tuples (any order)
+    uint2* dupLoose;         // [kDupLooseCap][maxCellLists] their loose tuples, ascending, and |tip|
+    uint32_t* dupOwner;      // [maxTuples] the lowest of them that has the tuple loose
+    uint8_t* dupCount;       // [maxCellLists] the number of them, 255 if more; 0 once the cell is done
     uint32_t* tupleOff;      // [maxTuples + 64]
     uint16_t* tupleBins;     // [5 * maxTuples]
     uint32_t* tupleCells;    // [4 * maxTuples] cells of a tuple (0xffffffff past the end)

@@ -1,0 +1,39 @@
+// Self-test entry point of the fast duplicate remover (csrc/kern_classify.hip) on track
+// lists the caller makes up, for tests/test_gpu_duplicates.py.  Test support only; the
+// reconstruction library does not load it.
+#include "../../pixeltrack-standalone_amd/csrc/kern_classify.hip"
+
+// One event: nMulti cells (any order) with counts[k] <= 48 ascending tuple indices each at
+// lists[48 k], the tuples' qualities and impact parameters.  All pointers are device
+// arrays; the caller's scratch: cellSlot[nCells] i32, cellCount[nCells] u16, dupCells
+// [nMulti] u32, dupLoose[6 nMulti] u64, dupCount[nMulti] u8, dupOwner[nTuples] u32 all ones,
+// counts one CACounts.  quality
+// and each of the five rows of state have nTuples entries, a multiple of 32.
+extern "C" int pxs_fast_duplicates(uint32_t nTuples, uint32_t nCells, uint32_t nMulti, uint32_t* cells,
+                                   int32_t* cellSlot, uint16_t* cellCount, uint32_t* lists, uint8_t* quality,
+                                   float* state, uint32_t* dupCells, uint2* dupLoose, uint8_t* dupCount, uint32_t* dupOwner,
+                                   void* counts, uint32_t blocks) {
+  using namespace pxg;
+  CACounts c{};
+  c.nMulti = nMulti;
+  c.nTuples = nTuples;
+  c.nCells = nCells;
+  if (hipMemcpy(counts, &c, sizeof(c), hipMemcpyHostToDevice) != hipSuccess)
+    return -1;
+  CAPool ca{};
+  ca.caps = {nCells, nTuples, nTuples, nTuples, nMulti, 128};
+  ca.cnt = static_cast<CACounts*>(counts);
+  ca.multiCells = cells;
+  ca.trSlot = cellSlot;
+  ca.trCount = cellCount;
+  ca.trPool = lists;
+  ca.quality = quality;
+  ca.state = state;
+  ca.dupCells = dupCells;
+  ca.dupLoose = dupLoose;
+  ca.dupCount = dupCount;
+  ca.dupOwner = dupOwner;
+  dupActiveKernel<<<dim3(blocks, 1), kCaBlock>>>(ca);
+  fastDuplicateKernel<<<1, kEventBlock>>>(ca);
+  return hipDeviceSynchronize() == hipSuccess && hipGetLastError() == hipSuccess ? 0 : -1;
+}

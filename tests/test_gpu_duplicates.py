@@ -1,0 +1,77 @@
+"""The fast duplicate remover's rounds (csrc/kern_classify.hip) on made-up track lists
+against the serial loop (CAHitNtupletGeneratorKernelsImpl.h:151-189): cells in ascending
+order, each keeping its loose tuple of smallest |tip|.  The lists reach what events seldom
+do: more loose tuples in a cell than the kernel keeps beside it, more tuples than the
+slot table has entries, long chains of cells that each wait for the one before, more cells
+than threads, tied impact parameters."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+from conftest import REPO
+
+pytestmark = pytest.mark.gpu
+LIB = os.path.join(REPO, "tests", "native", "libpxduplicates_selftest.so")
+BAD, DUP, LOOSE = 0, 1, 2
+
+
+def serial(cells, lists, quality, tip):
+    q = quality.copy()
+    for k in np.argsort(cells):
+        best, score = None, np.float32(10000)
+        for t in lists[k]:
+            if q[t] == LOOSE and abs(tip[t]) < score:
+                best, score = t, abs(tip[t])
+        for t in lists[k]:
+            if q[t] != BAD and t != best:
+                q[t] = DUP
+    return q
+
+
+@pytest.mark.parametrize("n_tuples,n_cells,width,loose", [
+    (1, 0, 0, 1.0),           # nothing to do
+    (40, 3, 2, 1.0),          # less than a wavefront
+    (500, 65, 48, 1.0),       # every list past what is kept beside a cell, all waiting on each other
+    (4000, 1500, 9, 0.5),     # lists on both sides of it; more cells than threads
+    (30000, 5000, 4, 0.7),
+    (100000, 20000, 3, 0.8),  # more tuples than slots
+])
+def test_rounds_match_the_serial_loop(n_tuples, n_cells, width, loose):
+    import torch
+    lib = C.CDLL(LIB)
+    vp, u32 = C.c_void_p, C.c_uint32
+    lib.pxs_fast_duplicates.argtypes = [u32, u32, u32] + [vp] * 11 + [u32]
+    rng = np.random.default_rng(n_tuples)
+    lists = [np.sort(rng.choice(n_tuples, size=rng.integers(2, width + 1), replace=False)) for _ in range(n_cells)]
+    if n_cells > 100:  # a chain: cell k shares a tuple with cell k + 1 only
+        lists[:50] = [np.array([k, k + 1]) for k in range(50)]
+    space = max(1, 3 * n_cells)
+    cells = rng.permutation(space)[:n_cells]
+    if n_cells > 100:
+        cells[:50] = np.sort(cells[:50])
+    quality = np.where(rng.random(n_tuples) < loose, LOOSE, rng.integers(0, 2, n_tuples)).astype(np.uint8)
+    tip = rng.choice(np.linspace(-0.4, 0.4, 97), n_tuples).astype(np.float32)  # ties among them
+    want = serial(cells, lists, quality, tip)
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+    slot, count = np.full(space, -1, np.int32), np.zeros(space, np.int16)
+    pool = np.zeros((max(1, n_cells), 48), np.int32)
+    for k, (c, l) in enumerate(zip(cells, lists)):
+        slot[c], count[c] = k, len(l)
+        pool[k, :len(l)] = l
+    stride = (n_tuples + 31) // 32 * 32
+    state = np.zeros((5, stride), np.float32)
+    state[1, :n_tuples] = tip
+    quality = np.append(quality, np.full(stride - n_tuples, BAD, np.uint8))
+    m = max(1, n_cells)
+    t = [dev(np.append(cells, 0).astype(np.int32)), dev(slot), dev(count), dev(pool), dev(quality), dev(state),
+         dev(np.zeros(m, np.int32)), dev(np.zeros(6 * m, np.int64)), dev(np.zeros(m, np.uint8)),
+         dev(np.full(stride, -1, np.int32)), dev(np.zeros(128, np.uint8))]
+    torch.cuda.synchronize()
+    assert lib.pxs_fast_duplicates(stride, space, n_cells, *[x.data_ptr() for x in t], 8) == 0
+    got = t[4].cpu().numpy()[:n_tuples]
+    assert np.array_equal(got, want), f"{(got != want).sum()} of {n_tuples} qualities differ"
