@@ -70,8 +70,8 @@ ROWS = {
 LABEL_ROW = {lab: row for row, (labs, _) in ROWS.items() for lab in labs}
 # device kernel symbol -> profiler label (several kernels make up "clusterize")
 KERNEL_LABEL = {
-    "decodeKernel": "decode", "moduleStartKernel": "moduleStarts", "clusterSmallKernel": "clusterize",
-    "clusterMediumKernel": "clusterize", "clusterBigKernel": "clusterize", "clusStartKernel": "clusterize",
+    "decodeKernel": "decode", "moduleStartKernel": "moduleStarts", "clusterRunsKernel": "clusterize",
+    "clusterBigKernel": "clusterize", "clusStartKernel": "clusterize",
     "hitsKernel": "hits",
     "phiBinnerKernel": "phiBinner", "doubletCountKernel": "doubletCount", "doubletScanKernel": "doubletScan",
     "doubletFillKernel": "doubletFill", "ohScanKernel": "outerHitScan", "ohFillKernel": "outerHitFill",

@@ -8,7 +8,7 @@
 // result depends only on the connected components, so any exact algorithm
 // gives the same labels; two are used here, picked per module run:
 //
-//   clusterSmallKernel  two module runs of at most 64 digis per wavefront
+//   clusterRunsKernel   on a wavefront, two module runs of at most 64 digis
 //                       (most modules at PU50 carry ~30: on the two halves when
 //                       both fit 32 lanes): a neighbour mask per lane from
 //                       shuffles, min-label propagation
@@ -18,15 +18,14 @@
 //                       The surviving clusters' extents and charges, which the
 //                       rec-hit stage needs, are accumulated in LDS on the way
 //                       and written once per cluster (ClusterExt).
-//                       Larger runs are listed per event in order by the
-//                       module-start scan.
-//   clusterMediumKernel runs of 65 to 256 digis, one wavefront each (a
-//   clusterBigKernel    workgroup of one wave), and the larger ones, a few
-//                       256-thread workgroups per event: pixels staged in LDS,
-//                       column histogram, lock-free union-find that hooks the
-//                       larger root under the smaller (so the root of a
-//                       component is its smallest index), roots numbered by a
-//                       workgroup scan.
+//                       Larger runs, listed per event in order by the
+//                       module-start scan, on a 256-thread workgroup each:
+//                       pixels staged in LDS, column histogram, lock-free
+//                       union-find that hooks the larger root under the smaller
+//                       (so the root of a component is its smallest index),
+//                       roots numbered by a workgroup scan.
+//   clusterBigKernel    the same for the runs of more than 1024 digis, whose
+//                       pixels take 51 KB of LDS.
 //   clusStartKernel     one workgroup per event: the clamped prefix over the
 //                       2000 cluster counts (SiPixelRawToClusterGPUKernel.cc:
 //                       464-506).
@@ -40,9 +39,10 @@ namespace pxg {
     constexpr int kWaves = kBlock / 64;
     constexpr uint32_t kNoPixel = 0xffffffffu;
     constexpr int kCols = kColsPerModule;  // 416
-    // workgroups per event for the runs of 65 to 256 digis (one wave each, ~4096 per
-    // launch) and for the larger ones (a few per event at most)
-    constexpr uint32_t kMediumWorkgroups = 4096, kMediumPerEventMax = 64, kBigPerEvent = 2;
+    // workgroups per event for the listed runs: about one per run at PU50 for a few
+    // events, as many as fill the device for many
+    constexpr uint32_t kMediumWorkgroups = 4096, kMediumPerEventMax = 512;
+    constexpr uint32_t kBigWorkgroups = 1024, kBigPerEventMin = 4, kBigPerEventMax = 96;
 
     __device__ __forceinline__ uint32_t findRoot(volatile uint32_t* parent, uint32_t x) {
       uint32_t p = parent[x];
@@ -81,13 +81,12 @@ namespace pxg {
     uint32_t parent[MAXPIX];  // union-find; later the cluster id
     uint32_t work[MAXPIX > 2 * kClusCap ? MAXPIX : 2 * kClusCap];  // column-sorted pixels; later charges/renumbering
     // column starts [0, kCols + 2) and fill cursors [kCols + 2, 2 kCols + 2); once the
-    // components are found, the cluster extents of a run of at most 256 digis
+    // components are found, the cluster extents of a run of at most kMediumRunMax digis
     uint32_t cols[2 * kCols + 2];
     uint32_t wsum[NT / 64];
   };
 
-  // one module run with a whole workgroup of NT threads (a run of up to MAXPIX digis;
-  // the largest runs, up to 4000 digis, on 256 threads)
+  // one module run of up to MAXPIX digis with a whole workgroup of NT threads
   template <int NT, uint32_t MAXPIX>
   __device__ void clusterRunWG(const Pool& p, uint32_t e, uint32_t k, RunLds<NT, MAXPIX>& L) {
     constexpr uint32_t kClusCap = RunLds<NT, MAXPIX>::kClusCap;
@@ -219,8 +218,8 @@ namespace pxg {
     }
 
     // ---- charge cut
-    int32_t* charge = reinterpret_cast<int32_t*>(work);                        // [kClusCap]
-    uint32_t* newId = work + kClusCap;                                         // [kClusCap]
+    uint32_t* newId = work;                                          // [kClusCap]
+    int32_t* charge = reinterpret_cast<int32_t*>(work + kClusCap);   // [kClusCap]
     for (uint32_t c = threadIdx.x; c < ncut; c += NT)
       charge[c] = 0;
     __syncthreads();
@@ -269,15 +268,16 @@ namespace pxg {
       p.moduleId[size_t(e) * kMaxModuleRanges + k] = me;
     }
 
-    // Runs of at most 256 digis also record each cluster's extent and charges for the
-    // rec-hit stage (ClusterExt, as the wavefront kernel does), accumulated with LDS
-    // atomics in the column area, which holds the nine fields of 92 clusters at a time
-    // (nearly always all of the run's).  Every cluster of such a run has pixels.
-    if constexpr (MAXPIX <= 256) {
+    // Each cluster's extent and charges for the rec-hit stage (ClusterExt, as the wavefront
+    // kernel records them), accumulated with LDS atomics in an area that is free here: the
+    // column lists (the nine fields of 92 clusters at a time, nearly always all of the
+    // run's), or past newId for the largest runs (330 clusters).  Every cluster has pixels.
+    {
       if (p.clExt && n > 0) {
-        const uint32_t nf = renumber ? kept : found;
-        constexpr uint32_t kChunk = (2 * kCols + 2) / 9;
-        uint32_t* ext = L.cols;  // field j of chunk cluster c at ext[j * kChunk + c]
+        const uint32_t nf = renumber ? kept : ncut;
+        constexpr bool kLarge = MAXPIX > 2 * kClusCap;
+        constexpr uint32_t kChunk = (kLarge ? MAXPIX - kClusCap : 2 * kCols + 2) / 9;
+        uint32_t* ext = kLarge ? work + kClusCap : L.cols;  // field j of chunk cluster c at ext[j * kChunk + c]
         auto finalId = [&](uint32_t i) -> uint32_t {
           if (sxy[i] == kNoPixel || parent[i] >= ncut)
             return 0xffffffffu;
@@ -502,22 +502,44 @@ namespace pxg {
     }
   }  // namespace
 
-  // kRuns (2) consecutive module runs per wavefront: on its two halves when both hold
-  // at most 32 digis (most at PU50), else one after the other on the whole wavefront
-  // (one run per wavefront for a few events, to fill the device); runs of more than
-  // 64 digis go to the work list of the workgroup kernel
+  // Runs of at most kMediumRunMax digis in one launch, so that the few longer ones run
+  // beside the many small ones: the first `medium` workgroups of an event take its listed
+  // runs of more than kWaveRunMax digis, one workgroup per run; the others kRuns (2)
+  // consecutive smaller runs per wavefront, on its two halves when both hold at most 32
+  // digis (most at PU50), else one after the other on the whole wavefront (one run per
+  // wavefront for a few events, to fill the device).  Bound: the latency of a run's chain
+  // of LDS passes (about 12 us for a run of 65 to 256 digis).  Against a launch each for the
+  // small runs, those of 65 to 256 digis on one wave each and the larger ones on two
+  // workgroups per event: one PU50 event 69 to 19 us, 128 of them 284 to 265 us, 12 PU200
+  // events 940 to 105 us.
   template <uint32_t kRuns>
-  __global__ void __launch_bounds__(kBlock) clusterSmallKernel(Pool p) {
-    __shared__ int32_t rowLds[kWaves][64];
-    __shared__ uint32_t extLds[kWaves][kExtFields][64];
+  __global__ void __launch_bounds__(kBlock) clusterRunsKernel(Pool p, uint32_t medium) {
+    struct SmallLds {
+      int32_t row[kWaves][64];
+      uint32_t ext[kWaves][kExtFields][64];
+    };
+    using MediumLds = RunLds<kBlock, kMediumRunMax>;
+    __shared__ union {
+      SmallLds small;
+      MediumLds medium;
+    } lds;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const LogicalBlock lb = logicalBlock();
-    const uint32_t k0 = kRuns * (lb.x * kWaves + wave);
     const uint32_t e = lb.y;
+    if (lb.x < medium) {
+      const uint32_t n = p.counts[e].nMediumRuns;
+      const uint32_t* list = p.bigList + size_t(e) * kMaxModuleRanges;
+      for (uint32_t i = lb.x; i < n; i += medium) {  // uniform per workgroup
+        clusterRunWG<kBlock, kMediumRunMax>(p, e, list[i], lds.medium);
+        __syncthreads();
+      }
+      return;
+    }
+    const uint32_t k0 = kRuns * ((lb.x - medium) * kWaves + wave);
     const EventDesc& ev = p.events[e];
     const uint32_t nModules = p.counts[e].nModules;
     if (k0 >= nModules)
-      return;  // uniform per wavefront; this kernel has no workgroup barrier
+      return;  // uniform per wavefront; no workgroup barrier from here on
     const uint32_t* ms = p.moduleStart + size_t(e) * kMaxModuleRanges;
     auto runOf = [&](uint32_t k, uint32_t& first) -> uint32_t {
       if (k >= nModules)
@@ -528,8 +550,8 @@ namespace pxg {
     };
     uint32_t f0 = 0, f1 = 0;
     const uint32_t n0 = runOf(k0, f0), n1 = kRuns > 1 ? runOf(k0 + 1, f1) : 0;
-    int32_t* row = rowLds[wave];
-    uint32_t(*ext)[64] = extLds[wave];
+    int32_t* row = lds.small.row[wave];
+    uint32_t(*ext)[64] = lds.small.ext[wave];
     if (n0 <= 32 && n1 <= 32) {
       const uint32_t half = lane >> 5;
       clusterRunLanes<32>(p, e, k0 + half, half ? f1 : f0, half ? n1 : n0, ev, row, ext, 32 * half,
@@ -540,21 +562,7 @@ namespace pxg {
     }
   }
 
-  // ---- larger module runs: each event's lists, their runs strided over its workgroups ----
-  // runs of 65 to 256 digis: one wavefront each (a workgroup of one wave, 7.4 KB of LDS)
-  constexpr uint32_t kMediumMaxPix = 256;
-  __global__ void __launch_bounds__(64) clusterMediumKernel(Pool p) {
-    __shared__ RunLds<64, kMediumMaxPix> L;
-    const uint32_t e = blockIdx.y;
-    const uint32_t n = p.counts[e].nMediumRuns;
-    const uint32_t* list = p.bigList + size_t(e) * kMaxModuleRanges;
-    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {  // uniform per workgroup
-      clusterRunWG<64, kMediumMaxPix>(p, e, list[i], L);
-      __syncthreads();
-    }
-  }
-
-  // runs of more than 256 digis (up to 4000), listed from the back of the event's list
+  // runs of more than kMediumRunMax digis (up to 4000), listed from the back of the event's list
   __global__ void __launch_bounds__(kBlock) clusterBigKernel(Pool p) {
     __shared__ RunLds<kBlock, kMaxPixInModule> L;
     const uint32_t e = blockIdx.y;
@@ -595,13 +603,16 @@ namespace pxg {
   }
 
   void launchClusterize(const Pool& p, uint32_t nEvents, hipStream_t s) {
+    if (nEvents == 0)
+      return;
+    const uint32_t med = std::max(1u, std::min(kMediumPerEventMax, kMediumWorkgroups / nEvents));
     if (nEvents < 8)
-      clusterSmallKernel<1><<<dim3((kMaxNumModules + kWaves - 1) / kWaves, nEvents), kBlock, 0, s>>>(p);
+      clusterRunsKernel<1><<<dim3(med + (kMaxNumModules + kWaves - 1) / kWaves, nEvents), kBlock, 0, s>>>(p, med);
     else
-      clusterSmallKernel<2><<<dim3((kMaxNumModules + 2 * kWaves - 1) / (2 * kWaves), nEvents), kBlock, 0, s>>>(p);
-    const uint32_t med = nEvents ? std::max(1u, std::min(kMediumPerEventMax, kMediumWorkgroups / nEvents)) : 1u;
-    clusterMediumKernel<<<dim3(med, nEvents), 64, 0, s>>>(p);
-    clusterBigKernel<<<dim3(kBigPerEvent, nEvents), kBlock, 0, s>>>(p);
+      clusterRunsKernel<2><<<dim3(med + (kMaxNumModules + 2 * kWaves - 1) / (2 * kWaves), nEvents), kBlock, 0, s>>>(
+          p, med);
+    const uint32_t big = std::max(kBigPerEventMin, std::min(kBigPerEventMax, kBigWorkgroups / nEvents));
+    clusterBigKernel<<<dim3(big, nEvents), kBlock, 0, s>>>(p);
     clusStartKernel<<<nEvents, 1024, 0, s>>>(p);
   }
 

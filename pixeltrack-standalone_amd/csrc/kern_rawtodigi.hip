@@ -322,8 +322,8 @@ namespace pxg {
       baseMod += uint32_t(total & 0xffffffffu);
       baseErr += uint32_t(total >> 32);
     }
-    // the runs the clusteriser's wavefront kernel cannot take, in order: those of 65 to
-    // 256 digis from the front of the event's list, the larger ones from its back
+    // the runs a wavefront of the clusteriser cannot take, in order: those of up to
+    // kMediumRunMax digis from the front of the event's list, the larger ones from its back
     __syncthreads();
     const uint32_t nMod = baseMod < kMaxNumModules ? baseMod : kMaxNumModules;
     uint32_t* bigList = p.bigList + size_t(e) * kMaxModuleRanges;
@@ -333,7 +333,7 @@ namespace pxg {
       uint32_t n = 0;
       if (k < nMod)
         n = (k + 1 < nMod ? moduleStart[2 + k] : nWords) - moduleStart[1 + k];
-      const bool med = n > 64 && n <= 256, big = n > 256;
+      const bool med = n > kWaveRunMax && n <= kMediumRunMax, big = n > kMediumRunMax;
       uint64_t total;
       const uint64_t at = wgExclusiveScan<kScanBlock>(uint64_t(med) | uint64_t(big) << 32, total, lds);
       if (med)

@@ -5,12 +5,11 @@
 //                   run would leave most lanes idle and make four times as many
 //                   latency chains), 64 for one event (more workgroups to fill
 //                   the device), one cluster per lane for the cluster position
-//                   estimate and the local -> global transform.  A run of at
-//                   most 256 digis (all but a few at PU50) takes its clusters'
-//                   extents and integer charges from the records the clustering
-//                   wrote (ClusterExt); a larger run accumulates them from its
-//                   digis with LDS atomics (exact in any order), G clusters per
-//                   pass.  The float
+//                   estimate and the local -> global transform, from the extents and
+//                   integer charges that the clustering recorded for runs of
+//                   any length (ClusterExt): passing twice over the digis of the
+//                   runs past 256 here took 381 of the 423 us of 12 PU200 events
+//                   and 40 of the 122 us of 128 PU50 events.  The float
 //                   arithmetic keeps the serial program's operation order and
 //                   the library is compiled without FMA contraction, so the
 //                   positions are bit-identical to the serial ones.
@@ -36,13 +35,6 @@ namespace pxg {
 
   namespace {
     constexpr int kBlock = 256;
-
-    // orders the wavefront's LDS accesses (lanes read what other lanes wrote)
-    __device__ __forceinline__ void waveSync() {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
 
     __device__ __forceinline__ uint32_t div52(uint32_t n) { return n / 52; }
     __device__ __forceinline__ bool bigX(uint32_t px) { return px == 79 || px == 80; }
@@ -103,7 +95,6 @@ namespace pxg {
   __global__ void __launch_bounds__(kBlock, 8) hitsKernel(DevConditions c, Pool p) {
     constexpr int kGroup = G;              // lanes per module run
     constexpr int kRuns = kBlock / kGroup;  // module runs per workgroup
-    constexpr int kChunk = kGroup;          // clusters per pass of a run
     const uint32_t lane = threadIdx.x % kGroup, run = threadIdx.x / kGroup;
     const LogicalBlock lb = logicalBlock();
     const uint32_t k = lb.x * kRuns + run;
@@ -136,11 +127,11 @@ namespace pxg {
     const uint32_t me = p.moduleId[mo + k];
     if (me >= kNumModules)
       return;
-    const uint32_t nclus = p.clusInModule[mo + me];
+    // past the capacity of a module the clusters have no digis
+    const uint32_t nclus = min(p.clusInModule[mo + me], kMaxClustersPerModule);
     if (nclus == 0)
       return;
     const uint32_t first = p.moduleStart[mo + 1 + k];
-    const uint32_t end = (k + 1 < nModules) ? p.moduleStart[mo + 2 + k] : ev.nWords;
     const uint32_t hitBase = p.clusModuleStart[mo + me];
     const size_t ho = size_t(e) * kMaxNumClusters;
     const CPEDetParams& det = c.cpeDet[me];
@@ -228,74 +219,11 @@ namespace pxg {
     };
 
     const uint32_t wo = ev.wordOffset;
-    if (end - first <= 256 && p.clExt) {
-      // a run of at most 256 digis: the clustering recorded its clusters' extents
-      const ClusterExt* ext = p.clExt + wo + first;
-      for (uint32_t ic = lane; ic < nclus; ic += kGroup) {
-        const ClusterExt x = ext[ic];
-        emit(ic, x.minRow, x.maxRow, x.minCol, x.maxCol, x.qfx, x.qlx, x.qfy, x.qly, x.qsum);
-      }
-      return;
-    }
-    // a larger run: cluster extents and charges from the digis, G clusters per pass
-    __shared__ uint32_t sMinRow[kRuns][kChunk], sMaxRow[kRuns][kChunk], sMinCol[kRuns][kChunk],
-        sMaxCol[kRuns][kChunk];
-    __shared__ int32_t sQsum[kRuns][kChunk], sQfx[kRuns][kChunk], sQlx[kRuns][kChunk], sQfy[kRuns][kChunk],
-        sQly[kRuns][kChunk];
-    uint32_t *minRow = sMinRow[run], *maxRow = sMaxRow[run], *minCol = sMinCol[run], *maxCol = sMaxCol[run];
-    int32_t *qsum = sQsum[run], *qfx = sQfx[run], *qlx = sQlx[run], *qfy = sQfy[run], *qly = sQly[run];
-
-    for (uint32_t start = 0; start < nclus; start += kChunk) {
-      const uint32_t nIn = min(uint32_t(kChunk), nclus - start);
-      if (lane < nIn) {
-        minRow[lane] = minCol[lane] = 0xffffffffu;
-        maxRow[lane] = maxCol[lane] = 0;
-        qsum[lane] = qfx[lane] = qlx[lane] = qfy[lane] = qly[lane] = 0;
-      }
-      waveSync();
-      for (uint32_t i = first + lane; i < end; i += kGroup) {
-        const uint32_t g = wo + i;
-        if (p.moduleInd[g] != me)
-          continue;  // invalid (or dropped) pixel
-        const int32_t cl = p.clus[g];
-        if (cl < int32_t(start) || cl >= int32_t(start + nIn))
-          continue;
-        const uint32_t j = uint32_t(cl) - start;
-        const uint32_t x = p.xx[g], y = p.yy[g];
-        atomicMin(&minRow[j], x);
-        atomicMax(&maxRow[j], x);
-        atomicMin(&minCol[j], y);
-        atomicMax(&maxCol[j], y);
-      }
-      waveSync();
-      for (uint32_t i = first + lane; i < end; i += kGroup) {
-        const uint32_t g = wo + i;
-        if (p.moduleInd[g] != me)
-          continue;
-        const int32_t cl = p.clus[g];
-        if (cl < int32_t(start) || cl >= int32_t(start + nIn))
-          continue;
-        const uint32_t j = uint32_t(cl) - start;
-        const uint32_t x = p.xx[g], y = p.yy[g];
-        const int32_t ch = p.adc[g];  // the 65535 clamp of the reference is a no-op on uint16
-        atomicAdd(&qsum[j], ch);
-        if (minRow[j] == x)
-          atomicAdd(&qfx[j], ch);
-        if (maxRow[j] == x)
-          atomicAdd(&qlx[j], ch);
-        if (minCol[j] == y)
-          atomicAdd(&qfy[j], ch);
-        if (maxCol[j] == y)
-          atomicAdd(&qly[j], ch);
-      }
-      waveSync();
-      for (uint32_t ic = lane; ic < nIn; ic += kGroup) {
-        if (hitBase + start + ic >= kMaxNumClusters)
-          break;
-        emit(start + ic, minRow[ic], maxRow[ic], minCol[ic], maxCol[ic], qfx[ic], qlx[ic], qfy[ic], qly[ic],
-             qsum[ic]);
-      }
-      waveSync();
+    // the clustering recorded the clusters' extents at the run's first digi + cluster id
+    const ClusterExt* ext = p.clExt + wo + first;
+    for (uint32_t ic = lane; ic < nclus; ic += kGroup) {
+      const ClusterExt x = ext[ic];
+      emit(ic, x.minRow, x.maxRow, x.minCol, x.maxCol, x.qfx, x.qlx, x.qfy, x.qly, x.qsum);
     }
   }
 

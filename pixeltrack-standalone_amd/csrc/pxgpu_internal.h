@@ -25,6 +25,10 @@ namespace pxg {
   constexpr int kDecodeBlock = 256;         // words per decode workgroup
   constexpr uint32_t kWordAlign = 256;      // event word offsets in a batch
   constexpr uint32_t kMaxModuleRanges = kMaxNumModules + 1;
+  // Module runs are clustered on a wavefront up to kWaveRunMax digis and by a workgroup
+  // beside them up to kMediumRunMax, where its 20 KB of LDS still leave a CU its 32 waves;
+  // longer ones (up to 4000 digis, 51 KB) in a launch of their own.
+  constexpr uint32_t kWaveRunMax = 64, kMediumRunMax = 1024;
 
   // status bits reported per event (a set bit never silently truncates a product)
   enum : uint32_t {
@@ -62,8 +66,8 @@ namespace pxg {
     uint32_t nClusters;
     uint32_t nErrors;
     uint32_t status;
-    uint32_t nMediumRuns;  // module runs of 65 to 256 digis, listed at the front of bigList
-    uint32_t nBigRuns;     // module runs of more than 256 digis, listed from the back of bigList
+    uint32_t nMediumRuns;  // module runs of 65 to kMediumRunMax digis, listed at the front of bigList
+    uint32_t nBigRuns;     // longer module runs, listed from the back of bigList
     uint32_t pad[2];
   };
 
@@ -103,8 +107,7 @@ namespace pxg {
     uint64_t* boundaryMask;  // [maxWords / 64]
     PixelErrorCompact* errorsSparse;  // [maxWords], error records at their word index
     PixelErrorCompact* errors;        // event e: errors[wordOffset[e] ...], word order
-    // [maxWords]: the clusters of a module run of at most 64 digis, found by the
-    // clustering, at the run's first digi + cluster id
+    // [maxWords]: the clusters of a module run at the run's first digi + cluster id
     ClusterExt* clExt;
     uint32_t* bigList;  // per event (stride kMaxModuleRanges): its module runs of more than 64 digis
     // clusters, per event

@@ -1,0 +1,63 @@
+"""Clustering and rec-hits of module runs at the lengths where the clusteriser changes its
+kernel (64 digis on a wavefront, 1024 beside them, 4000 in a launch of their own), sparse (a cluster per digi or two, more than an LDS chunk of cluster extents
+holds) and dense (few large clusters), against the oracle, bit for bit, for one event and
+for a batch."""
+import struct
+
+import numpy as np
+import pytest
+
+from test_gpu_stageAB import _compare
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = (1, 31, 32, 33, 63, 64, 65, 91, 255, 256, 257, 700, 1023, 1024, 1025, 3997, 3998)
+
+
+def _record(cond, lengths, rows, rng):
+    """A raw record with one run per length, each on a forward or outer barrel module of
+    its own: distinct pixels of the first `rows` rows of every ROC, a random charge."""
+    cab = cond["cabling"]
+
+    def table(k):
+        return cab[230400 * k:230400 * (k + 1)].view(np.uint32)
+
+    module = table(5)
+    feds = {}
+    free = [m for m in rng.permutation(np.arange(96, 1856)) if (module == m).any()]
+    for n in lengths:
+        m = free.pop()
+        slots = np.nonzero((module == m) & (cab[1382400:1382400 + 57600] == 0) & (cond["mod_to_unp"] == 0))[0]
+        fed, link, roc = slots // 384, table(1)[slots], table(2)[slots]
+        pix = rng.choice(len(slots) * 26 * 2 * rows, n, replace=False)
+        k, dcol, pxid = pix // (52 * rows), pix // (2 * rows) % 26, 2 + pix % (2 * rows)
+        words = (link[k] << 26) | (roc[k] << 21) | (dcol << 16) | (pxid << 8) | rng.integers(1, 256, n)
+        feds.setdefault(int(fed[0]), []).append(words.astype(np.uint32))
+    out = struct.pack("<I", len(feds))
+    for f, runs in sorted(feds.items()):
+        w = np.concatenate(runs)
+        w = np.append(w, np.zeros(len(w) % 2, np.uint32))
+        size = len(w) * 4 + 16
+        out += struct.pack("<IIQ", 1200 + f, size, 0x5 << 60 | (1200 + f) << 8) + w.tobytes() + \
+            struct.pack("<Q", 0xA << 60 | (size // 8) << 32)
+    return np.frombuffer(out, np.uint8)
+
+
+@pytest.mark.parametrize("rows", [16, 6])
+def test_runs_at_the_kernels_edges(conditions, oracle, gpu_ctx, gpu_stream, rows):
+    from pxtrack import gpu
+    rng = np.random.default_rng(rows)
+    raws = [_record(conditions, LENGTHS, rows, rng) for _ in range(8)]
+    inputs = [gpu.unpack_raw(r, conditions["fed_ids"]) for r in raws]
+    want = [oracle.process(r, upto=3) for r in raws]
+    assert max(o["clusInModule"].max() for o in want) > (300 if rows == 16 else 0)
+    g = gpu_stream.process(*inputs[0], upto=3)
+    assert g["status"] == 0
+    _compare(g, want[0], "one event")
+    s = gpu_ctx.stream(max_events=8, max_words=sum(len(w) for w, _ in inputs))
+    s.load(inputs)
+    s.run(0, 8, 3)
+    assert s.fetch_counts(0, 8) == 0
+    for e, o in enumerate(want):
+        _compare(s.event_products(e), o, f"event {e} of a batch")
+    s.close()
