@@ -54,7 +54,7 @@ ROWS = {
     "K4+K5 findClus+chargeCut (+K6 clamp scan)": (("clusterize",), lambda c: 10 * c["D"] + 14 * c["D"] + 16384),
     "K7 getHits": (("hits",), lambda c: 12 * c["D"] + 44 * c["H"]),
     "K8 layer start + phi binner": (("phiBinner",), lambda c: 6 * c["H"] + 5120),
-    "K9 doublets": (("doubletCount", "doubletScan", "doubletFill", "outerHitScan", "outerHitFill"),
+    "K9 doublets": (("doubletCount", "doubletScan", "doubletFill", "outerHitFill"),
                     lambda c: 14 * c["H"] + 12 * c["C"]),
     "K10 connect": (("connect",), lambda c: 8 * c["C"] + 16 * c["H"] + 4 * c["L"]),
     "K11 fishbone": (("fishbone",), lambda c: 12 * c["C"] + 16 * c["H"]),
@@ -74,8 +74,7 @@ KERNEL_LABEL = {
     "clusterBigKernel": "clusterize", "clusStartKernel": "clusterize",
     "hitsKernel": "hits",
     "phiBinnerKernel": "phiBinner", "doubletCountKernel": "doubletCount", "doubletScanKernel": "doubletScan",
-    "doubletFillKernel": "doubletFill", "ohScanKernel": "outerHitScan", "ohFillKernel": "outerHitFill",
-    "ohBuildKernel": "outerHitFill",
+    "doubletFillKernel": "doubletFill", "ohBuildKernel": "outerHitFill",
     "connectKernel": "connect", "fishboneKernel": "fishbone", "startMaskKernel": "startMask",
     "startCompactKernel": "startCompact", "ntupletCountKernel": "ntupletCount", "ntupletScanKernel": "ntupletScan",
     "ntupletFillKernel": "ntupletFill", "trackListAllocKernel": "trackListAlloc",

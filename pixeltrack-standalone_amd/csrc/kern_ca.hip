@@ -12,6 +12,8 @@
 // with gridDim.x workgroups; per-event scans run one workgroup per event.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "ca_device.h"
 
 namespace pxg {
@@ -237,11 +239,6 @@ namespace pxg {
       const uint32_t ntot = T.cum[kNumPairs - 1];
       const uint32_t total = wgScanArray<kEventBlock>(dOff, ntot, lds);
       const uint32_t nCells = min(total, ca.caps.maxDoublets);
-      const uint32_t nHits = T.layer[10];
-      // cleared for the following kernels
-      uint32_t* ohc = ca.ohCount + size_t(e) * kHitStride;
-      for (uint32_t h = threadIdx.x; h < nHits + 1; h += kEventBlock)
-        ohc[h] = 0;
       if (threadIdx.x == 0) {
         CACounts c{};
         c.nCells = nCells;
@@ -252,10 +249,7 @@ namespace pxg {
       }
     }
 
-    // kRank: each cell takes its place in its outer hit's list with an atomic on the
-    // hit's counter (the lists are then built by ohScanKernel and ohFillKernel); without
-    // it, ohBuildKernel builds the lists per event in LDS
-    template <int G, bool kRank>
+    template <int G>
     __global__ void __launch_bounds__(kCaBlock) doubletFillKernel(Pool p, CAPool ca) {
       const uint32_t e = logicalBlock().y;
       __shared__ PairTable T;
@@ -267,22 +261,18 @@ namespace pxg {
       const uint32_t ntot = T.cum[kNumPairs - 1];
       const uint32_t nCells = ca.cnt[e].nCells;
       const size_t cb = ca.cellBase(e);
-      uint32_t* ohc = ca.ohCount + size_t(e) * kHitStride;
       const uint64_t* dMask = ca.dMask + size_t(e) * 2 * kDoubletSlots;
       const uint32_t sub = laneId() % G;
       const uint64_t below = (1ull << sub) - 1;
-      if (!kRank) {
-        // the cells' state for connect and the fishbone, cleared in cell order on the
-        // whole grid, four cells per thread with one store per array (the per-event list
-        // build would do it on one CU); the cell stride of an event is a multiple of four,
-        // so the stores stay inside the event's arrays
-        static_assert(kCapsReference.maxDoublets % 4 == 0 && kCapsHighOccupancy.maxDoublets % 4 == 0, "cell stride");
-        for (uint32_t c = 4 * gridStart(); c < nCells; c += 4 * gridStride()) {
-          *reinterpret_cast<uint32_t*>(ca.cellFlags + cb + c) = 0;
-          *reinterpret_cast<uint32_t*>(ca.cellUsed + cb + c) = 0;
-          *reinterpret_cast<uint32_t*>(ca.nbCount + cb + c) = 0;
-          *reinterpret_cast<int4*>(ca.nbSlot + cb + c) = make_int4(-1, -1, -1, -1);
-        }
+      // the cells' state for connect and the fishbone, cleared in cell order on the whole
+      // grid, four cells per thread with one store per array; the cell stride of an event
+      // is a multiple of four, so the stores stay inside the event's arrays
+      static_assert(kCapsReference.maxDoublets % 4 == 0 && kCapsHighOccupancy.maxDoublets % 4 == 0, "cell stride");
+      for (uint32_t c = 4 * gridStart(); c < nCells; c += 4 * gridStride()) {
+        *reinterpret_cast<uint32_t*>(ca.cellFlags + cb + c) = 0;
+        *reinterpret_cast<uint32_t*>(ca.cellUsed + cb + c) = 0;
+        *reinterpret_cast<uint32_t*>(ca.nbCount + cb + c) = 0;
+        *reinterpret_cast<int4*>(ca.nbSlot + cb + c) = make_int4(-1, -1, -1, -1);
       }
       for (uint32_t j = groupSlotStart<G>(); j < ntot; j += groupSlotStride<G>()) {
         const uint32_t base = dOff[j];
@@ -293,8 +283,6 @@ namespace pxg {
           ca.cellInner[cb + c] = uint16_t(q.i);
           ca.cellOuter[cb + c] = uint16_t(oi);
           ca.cellPair[cb + c] = uint8_t(q.pairId);
-          if (kRank)
-            ca.ohRank[cb + c] = atomicAdd(&ohc[oi], 1u);
         };
         // the first 128 candidates: the count pass recorded their verdicts; the
         // r-th accepted one is the slot's r-th cell, written by lane r % G
@@ -326,134 +314,114 @@ namespace pxg {
     }
 
     // ---- outer-hit cell lists (GPUCACell::OuterHitOfCell, first maxCellsPerHit cells ascending) ----
-    __global__ void __launch_bounds__(kEventBlock) ohScanKernel(Pool p, CAPool ca) {
-      const uint32_t e = blockIdx.x;
+    // The cells of a layer pair are one contiguous range, and a hit is the outer hit only
+    // of cells of the pairs that end on its layer.  A workgroup therefore takes one part of
+    // one layer's hits and passes twice over the cells of that layer's pairs (an outer hit
+    // index each): LDS counts of its hits and a register count of the layer's lower hits
+    // give the offsets, the layers below it count as many cells as their pairs hold, and
+    // the second pass puts each cell at its place, taken with an LDS atomic (the consumers
+    // do not depend on the order within a list).
+    // Bound: latency of the two passes for a few events, the scattered stores of the second
+    // for many (17M cells of 128 PU50 events in 150 us).  The layers and parts spread an
+    // event over 9 to 72 CUs, for a re-read of the layer's 2 bytes per cell in each part.
+    // Against one workgroup per event over all cells (and, below 8 events, an atomic per
+    // cell in the doublet fill, a scan and a fill over the grid): one PU50 event 19 to 22 us
+    // with 6 less in the doublet fill, 16 events 124 to 32, 128 events 198 to 150, 12 PU200
+    // events 1235 to 241.  Eight cells per load gave nothing (225 to 241 us, 35 to 32).
+    constexpr uint32_t kOhSlice = 8192;  // hits counted at once: 32 KB
+    __global__ void __launch_bounds__(kEventBlock) ohBuildKernel(Pool p, CAPool ca, uint32_t parts) {
+      const LogicalBlock lb = logicalBlock();
+      const uint32_t e = lb.y;
+      const uint32_t layer = 1 + lb.x / parts, part = lb.x % parts;
+      __shared__ uint32_t cnt[kOhSlice];
       __shared__ uint32_t lds[kEventBlock / 64];
-      const uint32_t nHits = p.hitsLayerStart[size_t(e) * kLayerStartStride + 10];
-      uint32_t* cnt = ca.ohCount + size_t(e) * kHitStride;
-      uint32_t* off = ca.ohOff + size_t(e) * kHitStride;
-      uint32_t carry = 0;
-      for (uint32_t base = 0; base < nHits; base += kEventBlock) {
-        const uint32_t h = base + threadIdx.x;
-        const uint32_t v = h < nHits ? cnt[h] : 0;
-        uint32_t tot;
-        const uint32_t ex = wgExclusiveScan<kEventBlock>(v, tot, lds);
-        if (h < nHits)
-          off[h] = carry + ex;
-        carry += tot;
-      }
+      __shared__ PairTable T;
+      __shared__ uint32_t pairBeg[kNumPairs + 1];  // first cell of each pair
       if (threadIdx.x == 0)
-        off[nHits] = carry;
-    }
-
-    // each cell at its outer hit's offset plus the position the doublet fill's
-    // count gave it
-    __global__ void __launch_bounds__(kCaBlock) ohFillKernel(CAPool ca) {
-      const uint32_t e = logicalBlock().y;
+        loadPairTable(p.hitsLayerStart + size_t(e) * kLayerStartStride, T);
+      __syncthreads();
       const uint32_t nCells = ca.cnt[e].nCells;
-      const size_t cb = ca.cellBase(e);
-      const uint32_t* off = ca.ohOff + size_t(e) * kHitStride;
-      // four cells per iteration: their loads are issued together
-      const uint32_t stride = gridStride();
-      for (uint32_t c0 = gridStart(); c0 < nCells; c0 += 4 * stride) {
-        uint32_t h[4], hi[4], pos[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t c = c0 + u * stride;
-          if (c < nCells) {
-            h[u] = ca.cellOuter[cb + c];
-            hi[u] = ca.cellInner[cb + c];
-            pos[u] = ca.ohRank[cb + c];
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const uint32_t c = c0 + u * stride;
-          if (c < nCells) {
-            ca.ohCells[cb + off[h[u]] + pos[u]] = make_uint2(c, hi[u] | h[u] << 16);
-            ca.cellFlags[cb + c] = 0;
-            ca.cellUsed[cb + c] = 0;
-            ca.nbSlot[cb + c] = -1;
-            ca.nbCount[cb + c] = 0;
-            ca.trSlot[cb + c] = -1;
-            ca.trCount[cb + c] = 0;
-          }
-        }
-      }
-    }
-
-    // The outer-hit lists of one event by one workgroup, with the counts in LDS: a global
-    // atomic per cell costs ~48 ns of device throughput at scattered addresses on this
-    // chip, an LDS atomic a few cycles of one CU.  Counts per hit are 16 bits, two to a
-    // word (a hit's cells come from the inner hits of at most the 48k of the event, so
-    // no count reaches 65536): the counts, a workgroup scan into the offsets, then each
-    // cell at its hit's offset plus its rank, taken with a second round of LDS atomics
-    // (the consumers do not depend on the order within a list).  The doublet fill has
-    // cleared the cells' state for the later stages.
-    __global__ void __launch_bounds__(kEventBlock) ohBuildKernel(Pool p, CAPool ca) {
-      const uint32_t e = blockIdx.x;
-      __shared__ uint32_t hist[kMaxNumClusters / 2];
-      __shared__ uint32_t lds[kEventBlock / 64];
-      const uint32_t nHits = p.hitsLayerStart[size_t(e) * kLayerStartStride + 10];
-      const uint32_t nCells = ca.cnt[e].nCells;
+      const uint32_t* dOff = ca.dOff + size_t(e) * (kDoubletSlots + 64);
+      if (threadIdx.x <= kNumPairs)
+        pairBeg[threadIdx.x] = min(dOff[threadIdx.x ? T.cum[threadIdx.x - 1] : 0], nCells);
+      __syncthreads();
       const size_t cb = ca.cellBase(e);
       uint32_t* off = ca.ohOff + size_t(e) * kHitStride;
-      const uint32_t nWords = (nHits + 1) / 2;
-      for (uint32_t w = threadIdx.x; w < nWords; w += kEventBlock)
-        hist[w] = 0;
-      __syncthreads();
-      constexpr uint32_t kU = 16;  // cells per thread and iteration: their loads are issued together
-      for (uint32_t c0 = threadIdx.x; c0 < nCells; c0 += kU * kEventBlock) {
-        uint32_t h[kU];
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) {
-          const uint32_t c = c0 + u * kEventBlock;
-          h[u] = c < nCells ? ca.cellOuter[cb + c] : 0xffffffffu;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kU; ++u)
-          if (h[u] != 0xffffffffu)
-            atomicAdd(&hist[h[u] >> 1], 1u << ((h[u] & 1) * 16));
+      if (lb.x == 0) {  // the first layer's hits are no cell's outer hit
+        for (uint32_t h = threadIdx.x; h < T.layer[1]; h += kEventBlock)
+          off[h] = 0;
+        if (threadIdx.x == 0)
+          off[T.layer[10]] = nCells;
       }
-      __syncthreads();
-      // offsets: each thread scans an even-sized run of hits (whole words), the runs in order
-      const uint32_t per = 2 * ((nWords + kEventBlock - 1) / kEventBlock);
-      const uint32_t h0 = min(threadIdx.x * per, nHits), h1 = min(h0 + per, nHits);
-      uint32_t sum = 0;
-      for (uint32_t h = h0; h < h1; ++h)
-        sum += (hist[h >> 1] >> ((h & 1) * 16)) & 0xffffu;
-      uint32_t total;
-      uint32_t run = wgExclusiveScan<kEventBlock>(sum, total, lds);
-      for (uint32_t h = h0; h < h1; ++h) {
-        off[h] = run;
-        run += (hist[h >> 1] >> ((h & 1) * 16)) & 0xffffu;
-      }
-      if (threadIdx.x == 0)
-        off[nHits] = total;
-      __syncthreads();
-      for (uint32_t w = h0 / 2; w < (h1 + 1) / 2; ++w)
-        hist[w] = 0;  // the counts become ranks
-      __syncthreads();
-      for (uint32_t c0 = threadIdx.x; c0 < nCells; c0 += kU * kEventBlock) {
-        uint32_t h[kU], hi[kU];
+      const uint32_t hits = T.layer[layer + 1] - T.layer[layer];
+      const uint32_t per = (hits + parts - 1) / parts;
+      const uint32_t p0 = T.layer[layer] + min(part * per, hits), p1 = T.layer[layer] + min((part + 1) * per, hits);
+      uint32_t lower = 0;  // cells ending on lower layers
+      for (int q = 0; q < kNumPairs; ++q)
+        lower += kPairOuter[q] < layer ? pairBeg[q + 1] - pairBeg[q] : 0;
+      // f(first cell, outer hits) over the cells of the pairs ending on the layer, eight per
+      // thread and iteration, their loads issued together
+      constexpr uint32_t kU = 8;
+      auto forCells = [&](auto&& f) {
+        for (int q = 0; q < kNumPairs; ++q) {
+          if (kPairOuter[q] != layer)
+            continue;
+          const uint32_t c1 = pairBeg[q + 1];
+          for (uint32_t c0 = pairBeg[q] + threadIdx.x; c0 < c1; c0 += kU * kEventBlock) {
+            uint32_t h[kU];
 #pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) {
-          const uint32_t c = c0 + u * kEventBlock;
-          h[u] = hi[u] = 0;
-          if (c < nCells) {
-            h[u] = ca.cellOuter[cb + c];
-            hi[u] = ca.cellInner[cb + c];
+            for (uint32_t u = 0; u < kU; ++u) {
+              const uint32_t c = c0 + u * kEventBlock;
+              h[u] = c < c1 ? ca.cellOuter[cb + c] : 0xffffffffu;
+            }
+            f(c0, h);
           }
         }
+      };
+      for (uint32_t h0 = p0; h0 < p1; h0 += kOhSlice) {
+        const uint32_t n = min(kOhSlice, p1 - h0);
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < n; i += kEventBlock)
+          cnt[i] = 0;
+        __syncthreads();
+        uint32_t below = 0;
+        forCells([&](uint32_t, const uint32_t(&h)[kU]) {
 #pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) {
-          const uint32_t c = c0 + u * kEventBlock;
-          if (c < nCells) {
-            const uint32_t sh = (h[u] & 1) * 16;
-            const uint32_t rank = (atomicAdd(&hist[h[u] >> 1], 1u << sh) >> sh) & 0xffffu;
-            ca.ohCells[cb + off[h[u]] + rank] = make_uint2(c, hi[u] | h[u] << 16);
+          for (uint32_t u = 0; u < kU; ++u) {
+            below += h[u] < h0;
+            if (h[u] - h0 < n)
+              atomicAdd(&cnt[h[u] - h0], 1u);
           }
+        });
+        uint32_t base;
+        wgExclusiveScan<kEventBlock>(below, base, lds);
+        base += lower;
+        // offsets: each thread a run of consecutive hits, the runs in order
+        const uint32_t run = (n + kEventBlock - 1) / kEventBlock;
+        const uint32_t i0 = min(threadIdx.x * run, n), i1 = min(i0 + run, n);
+        uint32_t sum = 0;
+        for (uint32_t i = i0; i < i1; ++i)
+          sum += cnt[i];
+        uint32_t total;
+        uint32_t at = base + wgExclusiveScan<kEventBlock>(sum, total, lds);
+        for (uint32_t i = i0; i < i1; ++i) {
+          const uint32_t k = cnt[i];
+          off[h0 + i] = at;
+          cnt[i] = at;  // the counts become places
+          at += k;
         }
+        __syncthreads();
+        forCells([&](uint32_t c0, const uint32_t(&h)[kU]) {
+          uint32_t hi[kU];
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u)
+            hi[u] = h[u] - h0 < n ? ca.cellInner[cb + c0 + u * kEventBlock] : 0;
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u)
+            if (h[u] - h0 < n)
+              ca.ohCells[cb + atomicAdd(&cnt[h[u] - h0], 1u)] =
+                  make_uint2(c0 + u * kEventBlock, hi[u] | h[u] << 16);
+        });
       }
     }
 
@@ -1390,22 +1358,15 @@ namespace pxg {
     l.t->e();                                    \
   } while (0)
 
-  // the doublets and the outer-hit lists: per event in LDS for batches of 8 or more
-  // events (one workgroup per event fills the device), with per-cell atomics across
-  // the grid for smaller ones
   template <int G>
   void doubletKernels(const CALaunch& l) {
     const dim3 g(l.blocks, l.nEvents);
     PXG_K("doubletCount", doubletCountKernel<G>, g, kCaBlock, *l.p, *l.ca);
     PXG_K("doubletScan", doubletScanKernel, l.nEvents, kEventBlock, *l.p, *l.ca);
-    if (l.nEvents >= kListsInLdsMinEvents) {
-      PXG_K("doubletFill", (doubletFillKernel<G, false>), g, kCaBlock, *l.p, *l.ca);
-      PXG_K("outerHitFill", ohBuildKernel, l.nEvents, kEventBlock, *l.p, *l.ca);
-    } else {
-      PXG_K("doubletFill", (doubletFillKernel<G, true>), g, kCaBlock, *l.p, *l.ca);
-      PXG_K("outerHitScan", ohScanKernel, l.nEvents, kEventBlock, *l.p, *l.ca);
-      PXG_K("outerHitFill", ohFillKernel, g, kCaBlock, *l.ca);
-    }
+    PXG_K("doubletFill", doubletFillKernel<G>, g, kCaBlock, *l.p, *l.ca);
+    // as many parts per layer as leave every CU about three workgroups
+    const uint32_t parts = std::max(1u, std::min(8u, 768 / ((kNumLayers - 1) * l.nEvents)));
+    PXG_K("outerHitFill", ohBuildKernel, dim3((kNumLayers - 1) * parts, l.nEvents), kEventBlock, *l.p, *l.ca, parts);
   }
 
   void launchDoublets(const CALaunch& l) {

@@ -108,12 +108,10 @@ namespace pxg::detail {
     f(ca.cellPair, D);
     f(ca.cellFlags, D);
     f(ca.cellUsed, D);
-    f(ca.ohCount, HS);
     f(ca.ohOff, HS);
     f(ca.ohCells, D);
     f(ca.startCells, D);
     f(ca.nbSlot, D);
-    f(ca.ohRank, D);
     f(ca.nbCount, D);
     f(ca.nbPool, L * kCaMaxNeighbors);
     f(ca.startMask, E * (ca.caps.maxDoublets / 64 + 64));
@@ -221,12 +219,10 @@ namespace pxg::detail {
     v.cellPair += D;
     v.cellFlags += D;
     v.cellUsed += D;
-    v.ohCount += H;
     v.ohOff += H;
     v.ohCells += D;
     v.startCells += D;
     v.nbSlot += D;
-    v.ohRank += D;
     v.nbCount += D;
     v.nbPool += L * kCaMaxNeighbors;
     v.startMask += size_t(first) * (c.caps.maxDoublets / 64 + 64);

@@ -136,7 +136,6 @@ namespace pxg {
   constexpr uint32_t kHitStride = kMaxNumClusters + 64;      // per-event stride of per-hit offset arrays
   constexpr uint32_t kCaBlock = 256;                         // workgroup of the grid-stride CA kernels
   constexpr uint32_t kEventBlock = 1024;                     // workgroup of the per-event kernels
-  constexpr uint32_t kListsInLdsMinEvents = 8;               // batches this large build lists per event in LDS
   // vertex clustering algorithms (gpuVertexFinder.h:46-60; density is the reference's default)
   enum : int { kVertexDensity = 0, kVertexDBSCAN = 1, kVertexIterative = 2 };
   constexpr uint32_t kDupLooseCap = 6;                       // loose tuples kept per cell for the duplicate remover
@@ -197,12 +196,10 @@ namespace pxg {
     uint8_t* cellPair;
     uint8_t* cellFlags;      // bit1 killed
     uint8_t* cellUsed;       // [maxDoublets] 1: the cell has a neighbour or is one
-    uint32_t* ohCount;       // [kHitStride] cells per outer hit, then fill cursors
     uint32_t* ohOff;         // [kHitStride]
     uint2* ohCells;          // [maxDoublets] cells by outer hit (fill order): x cell, y inner hit | outer hit << 16
     uint32_t* startCells;    // [maxDoublets] start cells of the ntuplet walk, ascending
     int32_t* nbSlot;         // [maxDoublets] neighbour list slot (-1 none, -2 store full)
-    uint32_t* ohRank;        // [maxDoublets] position of the cell in its outer hit's list
     uint8_t* nbCount;        // [maxDoublets] neighbours stored (<= 36)
     uint32_t* nbPool;        // [maxCellLists * 36]
     uint64_t* startMask;     // [maxDoublets / 64 + 64] start cells of the ntuplet walk
