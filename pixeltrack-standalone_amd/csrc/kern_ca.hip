@@ -1150,18 +1150,25 @@ namespace pxg {
         for (uint32_t i = threadIdx.x; i < n; i += kEventBlock)
           cnt[i] = 0;
         __syncthreads();
-        auto inSlice = [&](uint32_t c) { return c != 0xffffffffu && c - c0 < n; };
-        for (uint32_t t = threadIdx.x; t < nT; t += kEventBlock) {
-          const uint4 c = cells4[t];
-          if (inSlice(c.x))
-            atomicAdd(&cnt[c.x - c0], 1u);
-          if (inSlice(c.y))
-            atomicAdd(&cnt[c.y - c0], 1u);
-          if (inSlice(c.z))
-            atomicAdd(&cnt[c.z - c0], 1u);
-          if (inSlice(c.w))
-            atomicAdd(&cnt[c.w - c0], 1u);
-        }
+        // f(cell - c0, tuple) over the tuples' cells in the slice (0xffffffff, no cell, is in
+        // none), four tuples per thread in flight
+        auto forSlice = [&](auto&& f) {
+          constexpr uint32_t kU = 4;
+          for (uint32_t t0 = threadIdx.x; t0 < nT; t0 += kU * kEventBlock) {
+            uint4 c[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u) {
+              const uint32_t t = t0 + u * kEventBlock;
+              c[u] = t < nT ? cells4[t] : make_uint4(~0u, ~0u, ~0u, ~0u);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u)
+              for (const uint32_t x : {c[u].x, c[u].y, c[u].z, c[u].w})
+                if (x != 0xffffffffu && x - c0 < n)
+                  f(x - c0, t0 + u * kEventBlock);
+          }
+        };
+        forSlice([&](uint32_t i, uint32_t) { atomicAdd(&cnt[i], 1u); });
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < n; i += kEventBlock)
           if (cnt[i] == 0) {
@@ -1195,21 +1202,12 @@ namespace pxg {
           cnt[i] = (rank - 1) << 18;  // the list's rank in the workgroup above, tuples placed below
         }
         __syncthreads();
-        auto place = [&](uint32_t c, uint32_t t) {
-          if (!inSlice(c))
-            return;
-          const uint32_t v = atomicAdd(&cnt[c - c0], 1u);
+        forSlice([&](uint32_t i, uint32_t t) {
+          const uint32_t v = atomicAdd(&cnt[i], 1u);
           const uint32_t slot = sBase + (v >> 18), pos = v & 0x3ffffu;
           if (slot + 1 < ca.caps.maxCellLists && pos < kCaMaxCellTracks)
             pool[size_t(slot) * kCaMaxCellTracks + pos] = t;
-        };
-        for (uint32_t t = threadIdx.x; t < nT; t += kEventBlock) {
-          const uint4 c = cells4[t];
-          place(c.x, t);
-          place(c.y, t);
-          place(c.z, t);
-          place(c.w, t);
-        }
+        });
       }
       if (status)
         atomicOr(&ca.cnt[e].status, status);
@@ -1275,77 +1273,79 @@ namespace pxg {
     }
 
     // ---- a16 tuple multiplicity (kernel_countMultiplicity / fillMultiplicity) ----------
-    // One workgroup per event.  Within a size the serial fill leaves tuples in
-    // descending index order; each tuple's place is computed from its rank.
+    // One workgroup per event.  Within a size the serial fill leaves tuples in descending
+    // index order; each tuple's place is computed from its rank.  A walk is at most four
+    // cells deep, so the sizes are 3, 4 and 5, and the counts of all three share 64 bits:
+    // one workgroup scan ranks the 8192 tuples of a pass (eight consecutive ones per
+    // thread, their offsets and qualities in four loads).  Bound: latency, a pass takes
+    // about two memory round trips and the scan's barriers.  Against 1024 tuples per pass
+    // with counts per size and wave: one PU50 event 19 to 8 us, 12 PU200 events 237 to 65.
     __global__ void __launch_bounds__(kEventBlock) multiplicityKernel(Pool p, CAPool ca) {
       const uint32_t e = blockIdx.x;
-      __shared__ uint32_t binCount[8], binEnd[8], carry[8];
-      __shared__ uint32_t waveCnt[8][kEventBlock / 64];
+      __shared__ uint64_t lds[kEventBlock / 64];
+      constexpr uint32_t kV = 8, kBits = 21;
+      static_assert(kCapsReference.maxTuples < (1u << kBits) && kCapsHighOccupancy.maxTuples < (1u << kBits) &&
+                        kCapsReference.maxTuples % kV == 0 && kCapsHighOccupancy.maxTuples % kV == 0,
+                    "three counts in 64 bits, eight tuples per load");
       const uint32_t nT = ca.cnt[e].nTuples;
       const size_t tb = ca.tupleBase(e);
       const uint32_t* off = ca.tupleOff + ca.offBase(e);
       const uint8_t* q = ca.quality + tb;
       const uint32_t cap = ca.caps.maxTuplesMult;
-      const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-      if (threadIdx.x < 8) {
-        binCount[threadIdx.x] = 0;
-        carry[threadIdx.x] = 0;
-      }
-      __syncthreads();
-      auto binOf = [&](uint32_t t) -> int {
-        const uint32_t nh = off[t + 1] - off[t];
-        return (nh < 3 || nh > 7 || q[t] == kQualityDup) ? -1 : int(nh);
+      // the sizes of tuples [t0, t0 + 8), 0 for a tuple that is left out; the packed counts
+      auto sizes = [&](uint32_t t0, uint32_t(&nh)[kV]) -> uint64_t {
+        uint64_t sum = 0;
+        if (t0 < nT) {
+          const uint4 a = *reinterpret_cast<const uint4*>(off + t0), b = *reinterpret_cast<const uint4*>(off + t0 + 4);
+          const uint2 ql = *reinterpret_cast<const uint2*>(q + t0);
+          const uint32_t o[kV + 1] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, off[t0 + kV]};
+#pragma unroll
+          for (uint32_t u = 0; u < kV; ++u) {
+            const uint32_t n = o[u + 1] - o[u];
+            const bool dup = (((u < 4 ? ql.x : ql.y) >> (8 * (u % 4))) & 0xff) == kQualityDup;
+            nh[u] = t0 + u < nT && n >= 3 && n <= 5 && !dup ? n : 0;
+            sum += nh[u] ? 1ull << (kBits * (nh[u] - 3)) : 0;
+          }
+        }
+        return sum;
       };
-      for (uint32_t t = threadIdx.x; t < nT; t += kEventBlock) {
-        const int b = binOf(t);
-        if (b >= 0)
-          atomicAdd(&binCount[b], 1u);
+      uint64_t mine = 0, all;
+      for (uint32_t t0 = kV * threadIdx.x; t0 < nT; t0 += kV * kEventBlock) {
+        uint32_t nh[kV];
+        mine += sizes(t0, nh);
       }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (int b = 0; b < 8; ++b) {
-          s += binCount[b];
-          binEnd[b] = s;
-        }
+      wgExclusiveScan<kEventBlock>(mine, all, lds);
+      auto count = [](uint64_t v, uint32_t b) { return uint32_t(v >> (kBits * b)) & ((1u << kBits) - 1); };
+      const uint32_t end[3] = {count(all, 0), count(all, 0) + count(all, 1), count(all, 0) + count(all, 1) + count(all, 2)};
+      if (threadIdx.x < 9) {
         uint32_t* mo = ca.multOff + size_t(e) * 16;
-        for (int b = 0; b < 8; ++b)
-          mo[b] = min(binEnd[b] - binCount[b], cap);
-        mo[8] = min(s, cap);
-        ca.cnt[e].nMult = min(s, cap);
-        if (s > cap)
-          atomicOr(&ca.cnt[e].status, kCaMultiplicityOverflow);
+        const uint32_t b = threadIdx.x;  // first entry of size b
+        mo[b] = min(b <= 3 ? 0u : b == 4 ? end[0] : b == 5 ? end[1] : end[2], cap);
+        if (b == 8) {
+          ca.cnt[e].nMult = min(end[2], cap);
+          if (end[2] > cap)
+            atomicOr(&ca.cnt[e].status, kCaMultiplicityOverflow);
+        }
       }
-      __syncthreads();
       TupleIndex* mb = ca.multBins + size_t(e) * cap;
-      for (uint32_t base = 0; base < nT; base += kEventBlock) {
-        const uint32_t t = base + threadIdx.x;
-        const int b = t < nT ? binOf(t) : -1;
-        uint32_t below = 0;
-        for (int bb = 3; bb < 8; ++bb) {
-          const uint64_t m = __ballot(b == bb);
-          if (lane == 0)
-            waveCnt[bb][wid] = __popcll(m);
-          if (b == bb)
-            below = __popcll(m & ((1ull << lane) - 1));
-        }
-        __syncthreads();
-        if (b >= 0) {
-          uint32_t rank = carry[b] + below;
-          for (int w = 0; w < wid; ++w)
-            rank += waveCnt[b][w];
-          const uint32_t pos = binEnd[b] - 1 - rank;
+      uint64_t before = 0;  // tuples of each size in the earlier passes
+      for (uint32_t base = 0; base < nT; base += kV * kEventBlock) {
+        const uint32_t t0 = base + kV * threadIdx.x;
+        uint32_t nh[kV] = {0, 0, 0, 0, 0, 0, 0, 0};
+        const uint64_t sum = sizes(t0, nh);
+        uint64_t total;
+        uint64_t rank = before + wgExclusiveScan<kEventBlock>(sum, total, lds);
+#pragma unroll
+        for (uint32_t u = 0; u < kV; ++u) {
+          if (nh[u] == 0)
+            continue;
+          const uint32_t b = nh[u] - 3;
+          const uint32_t pos = (b == 0 ? end[0] : b == 1 ? end[1] : end[2]) - 1 - count(rank, b);
           if (pos < cap)
-            mb[pos] = t;
+            mb[pos] = t0 + u;
+          rank += 1ull << (kBits * b);
         }
-        __syncthreads();
-        if (threadIdx.x < 8 && threadIdx.x >= 3) {
-          uint32_t s = 0;
-          for (int w = 0; w < kEventBlock / 64; ++w)
-            s += waveCnt[threadIdx.x][w];
-          carry[threadIdx.x] += s;
-        }
-        __syncthreads();
+        before += total;
       }
     }
 

@@ -340,23 +340,28 @@ namespace pxg {
 
     // a22 hit -> tuple association of the loose tuples (HitToTuple, CAConstants.h:65), a
     // one-to-many container over the event's hits with the reference's capacity, built in
-    // LDS: workgroup (s, e) owns the hits [s * kH2tSlice, (s + 1) * kH2tSlice) of event e
-    // and passes twice over the event's loose tuples.  The first pass counts its hits'
-    // tuples with LDS atomics and the entries of lower hits in a register, so that the
-    // offsets (clamped to the capacity, as the container's) need no other workgroup; the
-    // second writes each entry at its hit's offset plus the rank an LDS atomic gives (the
-    // triplet cleaner sorts each hit's list).  An entry past the capacity is dropped.
-    constexpr uint32_t kH2tSlice = 16384;  // hits per workgroup: 64 KB of counts
+    // LDS: workgroup (s, e) owns the hits [s * slice, (s + 1) * slice) of event e and passes
+    // twice over the event's loose tuples.  The first pass counts its hits' tuples with LDS
+    // atomics and the entries of lower hits in a register, so that the offsets (clamped to
+    // the capacity, as the container's) need no other workgroup; the counts then become
+    // places, and the second pass takes each entry's place with an LDS atomic (the triplet
+    // cleaner sorts each hit's list).  An entry past the capacity is dropped.
+    // Bound: latency, so each thread has four tuples in flight: their qualities and offsets
+    // in one load each, then all their hits.  Against one tuple at a time and slices of
+    // 16384 hits for any batch: one PU50 event 44 to 19 us, 128 events 79 to 35, 12 PU200
+    // events 567 to 153.
+    constexpr uint32_t kH2tSlice = 16384;      // hits per workgroup at most: 64 KB of counts
+    constexpr uint32_t kH2tSliceSmall = 4096, kH2tSmallMaxEvents = 32;  // for a few events, to spread one over CUs
 
-    __global__ void __launch_bounds__(kEventBlock) hitToTupleBuildKernel(Pool p, CAPool ca) {
+    __global__ void __launch_bounds__(kEventBlock) hitToTupleBuildKernel(Pool p, CAPool ca, uint32_t slice) {
       const uint32_t s = blockIdx.x, e = blockIdx.y;
       __shared__ uint32_t cnt[kH2tSlice];
       __shared__ uint32_t lds[kEventBlock / 64];
       const uint32_t nHits = p.hitsLayerStart[size_t(e) * kLayerStartStride + 10];
-      const uint32_t h0 = s * kH2tSlice;
+      const uint32_t h0 = s * slice;
       if (h0 >= nHits && s > 0)
         return;  // uniform per workgroup; workgroup 0 always writes the end offset
-      const uint32_t n = h0 < nHits ? min(kH2tSlice, nHits - h0) : 0;
+      const uint32_t n = h0 < nHits ? min(slice, nHits - h0) : 0;
       const uint32_t nT = ca.cnt[e].nTuples;
       const size_t tb = ca.tupleBase(e);
       const uint32_t* toff = ca.tupleOff + ca.offBase(e);
@@ -365,21 +370,42 @@ namespace pxg {
       const uint32_t cap = ca.caps.maxHitToTuple;
       uint32_t* hoff = ca.h2tOff + size_t(e) * kHitStride;
       TupleIndex* bins = ca.h2tBins + size_t(e) * cap;
+      // f(tuple, hit) over the hits of the loose tuples; a tuple has at most five hits.  The
+      // strides of an event's arrays are multiples of four, and its offsets go on for 64
+      // entries past its tuples.
+      static_assert(kCapsReference.maxTuples % 4 == 0 && kCapsHighOccupancy.maxTuples % 4 == 0, "tuple stride");
+      auto forEntries = [&](auto&& f) {
+        constexpr uint32_t kU = 4, kMaxHits = 5;
+        for (uint32_t t0 = kU * threadIdx.x; t0 < nT; t0 += kU * kEventBlock) {
+          const uint32_t q4 = *reinterpret_cast<const uint32_t*>(q + t0);
+          const uint4 o4 = *reinterpret_cast<const uint4*>(toff + t0);
+          const uint32_t o[kU + 1] = {o4.x, o4.y, o4.z, o4.w, toff[t0 + kU]};
+          uint32_t h[kU][kMaxHits], nh[kU];
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u) {
+            nh[u] = t0 + u < nT && ((q4 >> (8 * u)) & 0xff) == kQualityLoose ? o[u + 1] - o[u] : 0;
+#pragma unroll
+            for (uint32_t j = 0; j < kMaxHits; ++j)
+              h[u][j] = j < nh[u] ? tbins[o[u] + j] : 0;
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u)
+#pragma unroll
+            for (uint32_t j = 0; j < kMaxHits; ++j)
+              if (j < nh[u])
+                f(t0 + u, h[u][j]);
+        }
+      };
       for (uint32_t i = threadIdx.x; i < n; i += kEventBlock)
         cnt[i] = 0;
       __syncthreads();
       uint32_t below = 0;
-      for (uint32_t t = threadIdx.x; t < nT; t += kEventBlock) {
-        if (q[t] != kQualityLoose)
-          continue;
-        for (uint32_t k = toff[t]; k < toff[t + 1]; ++k) {
-          const uint32_t h = tbins[k];
-          if (h < h0)
-            ++below;
-          else if (h - h0 < n)
-            atomicAdd(&cnt[h - h0], 1u);
-        }
-      }
+      forEntries([&](uint32_t, uint32_t h) {
+        if (h < h0)
+          ++below;
+        else if (h - h0 < n)
+          atomicAdd(&cnt[h - h0], 1u);
+      });
       uint32_t base;
       wgExclusiveScan<kEventBlock>(below, base, lds);  // base: the entries of the lower hits
       // offsets: each thread takes a run of consecutive hits, the runs in order
@@ -391,9 +417,10 @@ namespace pxg {
       uint32_t total;
       uint32_t run = base + wgExclusiveScan<kEventBlock>(mine, total, lds);
       for (uint32_t i = i0; i < i1; ++i) {
+        const uint32_t k = cnt[i];
         hoff[h0 + i] = min(run, cap);
-        run += cnt[i];
-        cnt[i] = 0;  // the counts become ranks
+        cnt[i] = run;
+        run += k;
       }
       if (h0 + n == nHits && threadIdx.x == 0) {
         hoff[nHits] = min(base + total, cap);
@@ -401,20 +428,13 @@ namespace pxg {
           atomicOr(&ca.cnt[e].status, kCaHitToTupleOverflow);
       }
       __syncthreads();
-      for (uint32_t t = threadIdx.x; t < nT; t += kEventBlock) {
-        if (q[t] != kQualityLoose)
-          continue;
-        for (uint32_t k = toff[t]; k < toff[t + 1]; ++k) {
-          const uint32_t h = tbins[k];
-          if (h - h0 >= n)
-            continue;
-          // hoff[h] is the unclamped offset unless it reached the capacity, where every
-          // entry of h is dropped: the entry is kept iff its place is below the capacity
-          const uint32_t pos = hoff[h] + atomicAdd(&cnt[h - h0], 1u);
-          if (pos < cap)
-            bins[pos] = TupleIndex(t);
-        }
-      }
+      forEntries([&](uint32_t t, uint32_t h) {
+        if (h - h0 >= n)
+          return;
+        const uint32_t pos = atomicAdd(&cnt[h - h0], 1u);
+        if (pos < cap)
+          bins[pos] = TupleIndex(t);
+      });
     }
 
     // sorts each hit's tuples (descending, the serial fill order) and runs the
@@ -492,8 +512,9 @@ namespace pxg {
   void launchHitToTuple(const CALaunch& l) {
     const dim3 g(l.blocks, l.nEvents);
     l.t->b("hitToTupleFill");
-    hitToTupleBuildKernel<<<dim3((kMaxNumClusters + kH2tSlice - 1) / kH2tSlice, l.nEvents), kEventBlock, 0, l.s>>>(
-        *l.p, *l.ca);
+    const uint32_t slice = l.nEvents <= kH2tSmallMaxEvents ? kH2tSliceSmall : kH2tSlice;
+    hitToTupleBuildKernel<<<dim3((kMaxNumClusters + slice - 1) / slice, l.nEvents), kEventBlock, 0, l.s>>>(
+        *l.p, *l.ca, slice);
     l.t->e();
     l.t->b("tripletCleaner");
     tripletCleanerKernel<<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca);
