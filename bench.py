@@ -84,7 +84,9 @@ KERNEL_LABEL = {
     "dupActiveKernel": "dupActive", "fastDuplicateKernel": "fastDuplicate", "hitToTupleCountKernel": "hitToTupleCount",
     "hitToTupleScanKernel": "hitToTupleScan", "hitToTupleFillKernel": "hitToTupleFill",
     "hitToTupleBuildKernel": "hitToTupleFill",
-    "tripletCleanerKernel": "tripletCleaner", "vertexKernel": "vertices",
+    "tripletCleanerKernel": "tripletCleaner", "vertexSelectKernel": "vertices",
+    "vertexSortKernel": "vertices", "vertexCountKernel": "vertices", "vertexLinkKernel": "vertices",
+    "vertexFitKernel": "vertices",
 }
 
 

@@ -153,11 +153,12 @@ namespace pxg::detail {
     f(ca.vPtt2, T);
     f(ca.vIv, T);
     f(ca.vTmp, T);
-    f(ca.vZs, T);
-    f(ca.vEs, T);
+    f(ca.vZE, T);
     f(ca.vNnS, T);
-    f(ca.vIzt, T);
+    f(ca.vMask, T / 64);
     f(ca.vTrk, T);
+    f(ca.vPerm, T);
+    f(ca.vTerm, T);
     f(ca.vOff, E * (kMaxVertices + 64));
   }
 
@@ -264,11 +265,12 @@ namespace pxg::detail {
     v.vPtt2 += T;
     v.vIv += T;
     v.vTmp += T;
-    v.vZs += T;
-    v.vEs += T;
+    v.vZE += T;
     v.vNnS += T;
-    v.vIzt += T;
+    v.vMask += T / 64;
     v.vTrk += T;
+    v.vPerm += T;
+    v.vTerm += T;
     v.vOff += E * (kMaxVertices + 64);
     return v;
   }

@@ -233,11 +233,13 @@ namespace pxg {
     TupleIndex* vItrk;       // [maxTuples] tuple index of each loaded track
     float *vZt, *vEzt2, *vPtt2;      // [maxTuples]
     int32_t *vIv, *vTmp;     // [maxTuples]
-    float *vZs, *vEs;        // [maxTuples]: z and its error of the tracks in z-bin order
+    float2* vZE;             // [maxTuples]: z and its error of the tracks in z-bin order
     int32_t* vNnS;           // [maxTuples]: neighbour counts in z-bin order
-    uint8_t* vIzt;           // [maxTuples]
-    uint32_t* vTrk;          // [maxTuples]: tracks by vertex, ascending within a vertex
-    uint32_t* vOff;          // [kMaxVertices + 64]
+    uint64_t* vMask;         // [maxTuples / 64]: the tuples that are tracks for the vertex finder
+    uint32_t* vTrk;          // [maxTuples]: tracks by z bin, descending within a bin
+    uint32_t* vPerm;         // [maxTuples]: tracks by vertex, ascending within a vertex
+    float2* vTerm;           // [maxTuples]: terms of the vertices' sums, in that order
+    uint32_t* vOff;          // [kMaxVertices + 64]: starts of the z bins
 
     // per-event strides
     __host__ __device__ size_t cellBase(uint32_t e) const { return size_t(e) * caps.maxDoublets; }
