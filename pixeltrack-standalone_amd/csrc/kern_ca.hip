@@ -680,21 +680,29 @@ namespace pxg {
     // A cell seen from the list's hit: its inner hit relative to that hit.
     struct RowCell {
       uint32_t c;
-      uint32_t det;      // detInd of the inner hit; bit 16: the cell is used
+      uint32_t det;      // detInd of the inner hit
       float x, y, z, n;  // inner hit minus the list's hit, squared norm
     };
 
-    // lists that the wave's 64 positions touch, staged whole (up to kFbWindow entries, a
-    // launch-shape knob: 128, 256 or 384; at 256 six workgroups fit a CU); a wave whose
-    // lists span more reads them from memory
+    // A wavefront takes the lists that start among `span` consecutive list positions and
+    // stages their used cells in LDS (about one in seven; the others neither kill nor are
+    // killed), up to kFbWindow of them (a launch-shape knob: 128, 256 or 384), then runs a
+    // row per lane over the staged cells of its list.  Lists with more used cells than that,
+    // or longer than maxCellsPerHit, are read from memory.
+    // Bound: the gathers of the cells and their hits.  Staging every cell and running a row
+    // per list position, with six lanes of seven idle, took 225 us for 128 PU50 events
+    // (now 125) and 560 for 12 PU200 events (175).  A span of 256 gives a wavefront's lanes
+    // about 40 rows; a few events leave CUs idle with it (one PU50 event 16 us) and take 64
+    // (9.5; the kernel before took 9.4).
+    constexpr uint32_t kFbSpan = 256, kFbSpanFew = 64, kFbFewEvents = 8;
     template <bool kCheckTrack, uint32_t kFbWindow>
-    __global__ void __launch_bounds__(kCaBlock) fishboneKernel(Pool p, CAPool ca) {
+    __global__ void __launch_bounds__(kCaBlock) fishboneKernel(Pool p, CAPool ca, uint32_t span) {
       const uint32_t e = logicalBlock().y;
       const HitView H = hitsOf(p, e);
       if (H.layerStart[10] < 2)
         return;
-      // per wave: every cell of the lists its positions belong to, as seen from its
-      // list's hit (direction, squared norm; cell, detInd | used << 16)
+      // per wave: the used cells of its lists, as seen from their list's hit (direction,
+      // squared norm; cell, detInd | list's hit << 16)
       __shared__ float4 sDir[kCaBlock / 64][kFbWindow];
       __shared__ uint2 sCell[kCaBlock / 64][kFbWindow];
       const uint32_t nCells = ca.cnt[e].nCells;
@@ -703,13 +711,11 @@ namespace pxg {
       const uint2* cells = ca.ohCells + cb;
       const uint8_t* used = ca.cellUsed + cb;
       const uint16_t* trCount = ca.trCount + cb;
-      auto isUsed = [&](uint32_t c) {
-        return used[c] && (!kCheckTrack || trCount[c] > 0);
-      };
+      const uint32_t cap = ca.caps.maxCellsPerHit;
+      auto isUsed = [&](uint32_t c) { return used[c] && (!kCheckTrack || trCount[c] > 0); };
       // a list entry seen from its own list's hit
-      auto entry = [&](uint32_t k) {
+      auto entry = [&](const uint2& rec) {
         RowCell d;
-        const uint2 rec = cells[k];
         d.c = rec.x;
         const uint32_t hj = rec.y & 0xffff;
         const float4 ph = H.pos[rec.y >> 16];
@@ -718,102 +724,125 @@ namespace pxg {
         d.y = pj.y - ph.y;
         d.z = pj.z - ph.z;
         d.n = d.x * d.x + d.y * d.y + d.z * d.z;
-        d.det = uint32_t(H.detInd[hj]) | (isUsed(d.c) << 16);
+        d.det = H.detInd[hj];
         return d;
+      };
+      // the row of cell `me` over n cells of its list (get(k): the k-th; take(d): whether it
+      // takes part).  One pass finds the aligned later cells and the first closer one among
+      // them, which kills `me`; the aligned cells before that one are killed (several rows
+      // may kill a cell: they store the same byte).
+      auto row = [&](const RowCell& me, uint32_t n, uint32_t limit, auto get, auto take) {
+        auto aligned = [&](const RowCell& d) {
+          const float cos12 = me.x * d.x + me.y * d.y + me.z * d.z;
+          return me.det != d.det && cos12 * cos12 >= 0.99999f * me.n * d.n;
+        };
+        uint32_t killer = limit;
+        uint64_t alignedMask = 0;  // of the first 64 cells
+        for (uint32_t k = 0; k < n; ++k) {
+          const RowCell d = get(k);
+          if (d.c <= me.c || d.c >= limit || !take(d) || !aligned(d))
+            continue;
+          if (me.n > d.n && d.c < killer)
+            killer = d.c;
+          if (k < 64)
+            alignedMask |= 1ull << k;
+        }
+        for (uint64_t m = alignedMask; m; m &= m - 1) {
+          const uint32_t cj = get(__ffsll((unsigned long long)m) - 1).c;
+          if (cj < killer)
+            ca.cellFlags[cb + cj] |= 2;
+        }
+        for (uint32_t k = 64; k < n; ++k) {  // the others: second pass
+          const RowCell d = get(k);
+          if (d.c <= me.c || d.c >= killer || !take(d) || !aligned(d))
+            continue;
+          ca.cellFlags[cb + d.c] |= 2;
+        }
+        if (killer != limit)
+          ca.cellFlags[cb + me.c] |= 2;
+      };
+      // the row of a used cell over its whole list in memory; with more than maxCellsPerHit
+      // cells only that many lowest indices take part
+      auto rowFromMemory = [&](const RowCell& me, uint32_t h) {
+        const uint32_t b = off[h], n = off[h + 1] - b;
+        uint32_t limit = 0xffffffffu;
+        if (n > cap) {
+          if (!listedInOuterHit(cells, b, n, me.c, cap))
+            return;
+          for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t c = cells[b + k].x;
+            uint32_t rank = 0;
+            for (uint32_t m = 0; m < n; ++m)
+              rank += cells[b + m].x < c;
+            if (rank == cap)
+              limit = c;
+          }
+        }
+        row(me, n, limit, [&](uint32_t k) { return entry(cells[b + k]); },
+            [&](const RowCell& d) { return isUsed(d.c); });
       };
       const uint32_t lane = laneId(), wave = threadIdx.x / 64;
       float4* wDir = sDir[wave];
       uint2* wCell = sCell[wave];
-      for (uint32_t pos0 = gridStart() - lane; pos0 < nCells; pos0 += gridStride()) {  // uniform per wave
-        const uint32_t pos = pos0 + lane;
-        uint32_t b = 0, n = 0;
-        if (pos < nCells) {
-          const uint32_t h = cells[pos].y >> 16;
-          b = off[h];
-          n = off[h + 1] - b;
-        }
-        // the window: from the first list's start to the last list's end
-        const uint32_t last = min(63u, nCells - 1 - pos0);
-        const uint32_t wb = __shfl(b, 0);
-        const uint32_t we = __shfl(b + n, int(last));
-        const bool staged = we - wb <= kFbWindow;
-        if (staged) {
-          for (uint32_t k = lane; k < we - wb; k += 64) {
-            const RowCell d = entry(wb + k);
-            wDir[k] = make_float4(d.x, d.y, d.z, d.n);
-            wCell[k] = make_uint2(d.c, d.det);
+      const uint32_t spans = (nCells + span - 1) / span;
+      for (uint32_t s = waveStart(); s < spans; s += waveStride()) {
+        const uint32_t pos0 = s * span, last = min(pos0 + span, nCells) - 1;
+        const uint32_t h0 = cells[pos0].y >> 16;
+        const uint32_t ws = off[h0] == pos0 ? pos0 : off[h0 + 1], we = off[(cells[last].y >> 16) + 1];
+        uint32_t n = 0;
+        constexpr uint32_t kU = 4;  // list positions per lane and iteration: their loads are issued together
+        for (uint32_t k0 = ws; k0 < we; k0 += 64 * kU) {
+          uint2 rec[kU];
+          bool in[kU];
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u) {
+            const uint32_t k = k0 + 64 * u + lane;
+            rec[u] = k < we ? cells[k] : make_uint2(0, 0);
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u)
+            in[u] = k0 + 64 * u + lane < we && isUsed(rec[u].x);
+#pragma unroll
+          for (uint32_t u = 0; u < kU; ++u) {
+            const uint64_t m = __ballot(in[u]);
+            const uint32_t at = n + __popcll(m & lanesBelow());
+            n += __popcll(m);
+            if (in[u] && at < kFbWindow) {
+              const RowCell d = entry(rec[u]);
+              wDir[at] = make_float4(d.x, d.y, d.z, d.n);
+              wCell[at] = make_uint2(d.c, d.det | (rec[u].y & 0xffff0000u));
+            }
           }
         }
         waveLdsSync();
-        if (pos < nCells && n >= 2) {
-          const RowCell me = staged ? RowCell{wCell[pos - wb].x, wCell[pos - wb].y, wDir[pos - wb].x, wDir[pos - wb].y,
-                                              wDir[pos - wb].z, wDir[pos - wb].w}
-                                    : entry(pos);
-          const uint32_t ci = me.c;
-          if (me.det >> 16) {
-            // with more than maxCellsPerHit cells only that many lowest indices take part
-            const uint32_t cap = ca.caps.maxCellsPerHit;
-            uint32_t limit = 0xffffffffu;
-            bool listed = true;
-            if (n > cap) {
-              listed = listedInOuterHit(cells, b, n, ci, cap);
-              for (uint32_t k = 0; listed && k < n; ++k) {
-                const uint32_t c = cells[b + k].x;
-                uint32_t rank = 0;
-                for (uint32_t m = 0; m < n; ++m)
-                  rank += cells[b + m].x < c;
-                if (rank == cap)
-                  limit = c;
-              }
+        if (n <= kFbWindow) {
+          for (uint32_t r = lane; r < n; r += 64) {
+            const uint32_t key = wCell[r].y, h = key >> 16;
+            const float4 v = wDir[r];
+            const RowCell me{wCell[r].x, key & 0xffffu, v.x, v.y, v.z, v.w};
+            uint32_t lo = r, hi = r + 1;
+            while (lo > 0 && wCell[lo - 1].y >> 16 == h)
+              --lo;
+            while (hi < n && wCell[hi].y >> 16 == h)
+              ++hi;
+            if (hi - lo < 2)
+              continue;  // alone: kills none
+            if (we - ws > cap && off[h + 1] - off[h] > cap) {
+              rowFromMemory(me, h);
+              continue;
             }
-            auto fromMemory = [&](uint32_t k) { return entry(b + k); };
-            const uint32_t lo = b - wb;
-            auto fromLds = [&](uint32_t k) {
-              const float4 v = wDir[lo + k];
-              const uint2 c = wCell[lo + k];
-              return RowCell{c.x, c.y, v.x, v.y, v.z, v.w};
-            };
-            // one pass: the aligned later cells, and the first closer one among them
-            auto row = [&](auto get) {
-              uint32_t killer = limit;
-              uint64_t alignedMask = 0;  // list positions (lists of up to 64 cells)
-              for (uint32_t k = 0; k < n; ++k) {
-                const RowCell d = get(k);
-                if (d.c <= ci || d.c >= limit || !(d.det >> 16))
-                  continue;
-                const float cos12 = me.x * d.x + me.y * d.y + me.z * d.z;
-                if (!((me.det & 0xffff) != (d.det & 0xffff) && cos12 * cos12 >= 0.99999f * me.n * d.n))
-                  continue;
-                if (me.n > d.n && d.c < killer)
-                  killer = d.c;
-                if (k < 64)
-                  alignedMask |= 1ull << k;
-              }
-              // the aligned cells before the killer are killed (several rows may
-              // kill a cell: they store the same byte)
-              for (uint64_t m = alignedMask; m; m &= m - 1) {
-                const uint32_t cj = get(__ffsll((unsigned long long)m) - 1).c;
-                if (cj < killer)
-                  ca.cellFlags[cb + cj] |= 2;
-              }
-              for (uint32_t k = 64; k < n; ++k) {  // positions past 64: second pass
-                const RowCell d = get(k);
-                if (d.c <= ci || d.c >= killer || !(d.det >> 16))
-                  continue;
-                const float cos12 = me.x * d.x + me.y * d.y + me.z * d.z;
-                if ((me.det & 0xffff) != (d.det & 0xffff) && cos12 * cos12 >= 0.99999f * me.n * d.n)
-                  ca.cellFlags[cb + d.c] |= 2;
-              }
-              if (killer != limit)
-                ca.cellFlags[cb + ci] |= 2;
-            };
-            if (listed) {
-              if (staged)
-                row(fromLds);
-              else
-                row(fromMemory);
-            }
+            row(me, hi - lo, 0xffffffffu,
+                [&](uint32_t k) {
+                  const float4 w = wDir[lo + k];
+                  const uint2 c = wCell[lo + k];
+                  return RowCell{c.x, c.y & 0xffffu, w.x, w.y, w.z, w.w};
+                },
+                [](const RowCell&) { return true; });
           }
+        } else {
+          for (uint32_t k = ws + lane; k < we; k += 64)
+            if (isUsed(cells[k].x))
+              rowFromMemory(entry(cells[k]), cells[k].y >> 16);
         }
         waveLdsSync();
       }
@@ -1398,12 +1427,13 @@ namespace pxg {
   void fishboneLaunch(const CALaunch& l, const char* name) {
     const dim3 g(l.blocks, l.nEvents);
     l.t->b(name);
+    const uint32_t span = l.nEvents < kFbFewEvents ? kFbSpanFew : kFbSpan;
     if (l.fishboneWindow <= 128)
-      fishboneKernel<kCheckTrack, 128><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca);
+      fishboneKernel<kCheckTrack, 128><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca, span);
     else if (l.fishboneWindow <= 256)
-      fishboneKernel<kCheckTrack, 256><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca);
+      fishboneKernel<kCheckTrack, 256><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca, span);
     else
-      fishboneKernel<kCheckTrack, 384><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca);
+      fishboneKernel<kCheckTrack, 384><<<g, kCaBlock, 0, l.s>>>(*l.p, *l.ca, span);
     l.t->e();
   }
 

@@ -417,3 +417,24 @@ def test_products_do_not_depend_on_launch_shape(detector, oracle, gpu_ctx):
     assert shape["connect_stage"] in (128, 256, 512) and shape["fishbone_window"] in (128, 256, 384)
     with pytest.raises(RuntimeError):
         s.set_launch_shape(dict(connect_stage=200))
+
+
+@pytest.mark.parametrize("window,events", [(128, 8), (384, 8), (128, 3)])
+def test_fishbone_windows_on_noise_free_events(detector, oracle, gpu_ctx, window, events):
+    """Noise-free events, where most cells are used: up to 239 of 256 list positions, more
+    than the smallest window stages and less than the largest, for the spans of a few and of
+    many events per launch."""
+    from pxtrack import gpu
+    raws = [event(detector, "pu50", i, noise_frac=0.0, pu_lo=p, pu_hi=p)[0]
+            for i, p in enumerate((1, 5, 30, 2, 10, 5, 1, 20)[:events])]
+    unpacked = [gpu.unpack_raw(r, gpu_ctx.fed_ids) for r in raws]
+    s = gpu_ctx.stream(max_events=events, max_words=sum(w.size for w, _ in unpacked) + 256 * events)
+    s.set_launch_shape(dict(fishbone_window=window))
+    s.load(unpacked)
+    s.run(0, events, upto=5)
+    assert s.fetch_counts(0, events) == 0
+    for e, raw in enumerate(raws):
+        g = s.event_products(e, upto=5)
+        g.update(s.ca_internals(e, int(g["nHits"])))
+        compare_ca(oracle.process(raw, upto=5), g, f"window {window} event {e}")
+    s.close()
