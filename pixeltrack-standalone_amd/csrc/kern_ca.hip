@@ -483,6 +483,11 @@ namespace pxg {
       const uint32_t* off = ca.ohOff + size_t(e) * kHitStride;
       uint8_t* used = ca.cellUsed + cb;
       uint32_t* pool = ca.nbPool + size_t(e) * ca.caps.maxCellLists * kCaMaxNeighbors;
+      // hits are in module order: those of the modules below 96 and below 1184 come first
+      // (a gather of the inner hits' module ids took a quarter of the cache lines that a
+      // wavefront's setup touches)
+      const uint32_t* cms = p.clusModuleStart + size_t(e) * kMaxModuleRanges;
+      const uint32_t firstLayerEnd = cms[kLayerStart[1]], barrelEnd = cms[kModulesInBarrel];
       const uint32_t lane = laneId(), w = threadIdx.x >> 6;
       uint32_t status = 0, stored = 0;
       for (uint32_t pos0 = gridStart() - lane; pos0 < nCells; pos0 += gridStride()) {  // uniform per wave
@@ -506,8 +511,8 @@ namespace pxg {
           live = listedInOuterHit(ca.ohCells + cb, lb, ln, oc, ca.caps.maxCellsPerHit);
           p1 = H.pos[hi];
           p2 = H.pos[hm];
-          thetaCut = H.detInd[hm] < 1184 ? kCaThetaCutBarrel : kCaThetaCutForward;
-          dcut = H.detInd[hi] < 96 ? kCaDcaCutInner : kCaDcaCutOuter;
+          thetaCut = hm < barrelEnd ? kCaThetaCutBarrel : kCaThetaCutForward;
+          dcut = hi < firstLayerEnd ? kCaDcaCutInner : kCaDcaCutOuter;
         }
         // the outer layer of the cell's pair: the layer of its outer hit
         int lo = 0;
