@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <map>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/pxgpu.h"
@@ -37,17 +38,6 @@ namespace pxg::detail {
 using pxg::detail::fail;
 
 namespace {
-
-  template <typename T>
-  hipError_t devAlloc(T*& p, size_t n, std::vector<void*>& owned) {
-    void* q = nullptr;
-    hipError_t e = hipMalloc(&q, n * sizeof(T) + 256);
-    if (e == hipSuccess) {
-      owned.push_back(q);
-      p = static_cast<T*>(q);
-    }
-    return e;
-  }
 
   uint32_t alignUp(uint32_t v, uint32_t a) { return (v + a - 1) / a * a; }
 }  // namespace
@@ -168,7 +158,7 @@ namespace pxg::detail {
     ca.caps = caps;
     const uint32_t W = alignUp(maxWords, kWordAlign) + kWordAlign * maxEvents;
     size_t total = 0;
-    forEachArray(p, ca, maxEvents, W, [&](auto* ptr, size_t n) { total += n * sizeof(*ptr) + 256; });
+    forEachArray(p, ca, maxEvents, W, [&](auto* ptr, size_t n) { total += (n * sizeof(*ptr) + 511) / 256 * 256; });
     return total;
   }
 
@@ -460,9 +450,45 @@ namespace {
     return 0;
   }
 
+  // the staging buffer of the per-event entry points, for the longest event the pool takes
+  hipError_t allocStage(pxg_stream* s) {
+    const size_t words = std::min(s->wordCapacity, kMaxFedWords);
+    const size_t bytes = 4 * words + words / 2 + 64;
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&s->stage), bytes, hipHostMallocDefault);
+    if (e == hipSuccess)
+      e = hipHostGetDevicePointer(reinterpret_cast<void**>(&s->stageDev), s->stage, 0);
+    return e;
+  }
+
   void markLoaded(pxg_stream* s, uint32_t n) {
     s->nLoaded = n;
     std::fill(s->stagesRun.begin(), s->stagesRun.end(), uint8_t(0));
+  }
+
+  // the counters of a call's events to mapped host memory: one launch where a copy per array
+  // costs a launch and a copy's host work each
+  __global__ void __launch_bounds__(256) countsOutKernel(const uint32_t* a, uint32_t* hostA, uint32_t nA,
+                                                         const uint32_t* b, uint32_t* hostB, uint32_t nB) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nA)
+      hostA[i] = a[i];
+    else if (i - nA < nB)
+      hostB[i - nA] = b[i - nA];
+  }
+
+  // one event's words, FED ids and descriptor into the start of the pool, 16 bytes per lane
+  // from mapped host memory; the last lane of either array may go up to 12 bytes past its
+  // end, inside the pool's 256-word event slot and the staging buffer's padding
+  __global__ void __launch_bounds__(256) loadOneKernel(const uint4* words, uint4* dstWords, uint32_t nWords4,
+                                                       const uint4* fedIds, uint4* dstFedIds, uint32_t nFeds16,
+                                                       EventDesc* dst, EventDesc ev) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nWords4)
+      dstWords[i] = words[i];
+    else if (i - nWords4 < nFeds16)
+      dstFedIds[i - nWords4] = fedIds[i - nWords4];
+    if (i == 0)
+      *dst = ev;
   }
 
   // event blockIdx.y of the table: its words and FED ids from host memory into the pool
@@ -475,6 +501,14 @@ namespace {
       fedIds[g.wordOffset / 2 + i] = g.fedIds[i];
   }
 }  // namespace
+
+void pxg::detail::launchCountsOut(const EventCounts* counts, EventCounts* hostCounts, const CACounts* ca,
+                                  CACounts* hostCA, uint32_t n, hipStream_t s) {
+  const uint32_t nA = n * (sizeof(EventCounts) / 4), nB = ca ? n * (sizeof(CACounts) / 4) : 0;
+  countsOutKernel<<<(nA + nB + 255) / 256, 256, 0, s>>>(
+      reinterpret_cast<const uint32_t*>(counts), reinterpret_cast<uint32_t*>(hostCounts), nA,
+      reinterpret_cast<const uint32_t*>(ca), reinterpret_cast<uint32_t*>(hostCA), nB);
+}
 
 int pxg::detail::loadEvents(pxg_stream* s, uint32_t n, const pxg_raw_view* raws, const pxg_beamspot* bs,
                              uint32_t nBeamspots, bool sync) {
@@ -611,10 +645,25 @@ int pxg_stream_create_profile(pxg_context* ctx, uint32_t maxEvents, uint32_t max
   hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
   CAPool& ca = s->ca;
   ca.caps = profile == PXG_PROFILE_HIGH_OCCUPANCY ? kCapsHighOccupancy : kCapsReference;
-  forEachArray(p, ca, maxEvents, W, [&](auto*& ptr, size_t n) {
-    if (e == hipSuccess)
-      e = devAlloc(ptr, n, o);
-  });
+  // One allocation for the whole pool, its arrays 256-byte aligned in it with at least 256
+  // bytes between them: a hundred of their own take a hundred times as long.
+  size_t total = 0;
+  auto next = [&](size_t bytes) { return total += (bytes + 511) / 256 * 256; };
+  forEachArray(p, ca, maxEvents, W, [&](auto*& ptr, size_t n) { next(n * sizeof(*ptr)); });
+  next(PXG_N_COUNTERS * sizeof(*s->counters));
+  void* arena = nullptr;
+  if (e == hipSuccess)
+    e = hipMalloc(&arena, total);
+  if (e == hipSuccess) {
+    o.push_back(arena);
+    total = 0;
+    auto place = [&](auto*& ptr, size_t n) {
+      ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(static_cast<char*>(arena) + total);
+      next(n * sizeof(*ptr));
+    };
+    forEachArray(p, ca, maxEvents, W, place);
+    place(s->counters, PXG_N_COUNTERS);
+  }
   if (e == hipSuccess)
     e = hipHostMalloc(reinterpret_cast<void**>(&s->hostEvents), E * sizeof(EventDesc), hipHostMallocDefault);
   if (e == hipSuccess)
@@ -622,11 +671,15 @@ int pxg_stream_create_profile(pxg_context* ctx, uint32_t maxEvents, uint32_t max
   if (e == hipSuccess)
     e = hipHostMalloc(reinterpret_cast<void**>(&s->hostCA), E * sizeof(CACounts), hipHostMallocDefault);
   if (e == hipSuccess)
+    e = hipHostGetDevicePointer(reinterpret_cast<void**>(&s->hostCountsDev), s->hostCounts, 0);
+  if (e == hipSuccess)
+    e = hipHostGetDevicePointer(reinterpret_cast<void**>(&s->hostCADev), s->hostCA, 0);
+  if (e == hipSuccess && maxEvents == 1)  // a stream for the per-event entry points
+    e = allocStage(s);
+  if (e == hipSuccess)
     e = hipMemsetAsync(p.counts, 0, E * sizeof(EventCounts), s->stream);
   if (e == hipSuccess)
     e = hipMemsetAsync(ca.cnt, 0, E * sizeof(CACounts), s->stream);
-  if (e == hipSuccess)
-    e = devAlloc(s->counters, PXG_N_COUNTERS, o);
   if (e == hipSuccess)
     e = hipMemsetAsync(s->counters, 0, PXG_N_COUNTERS * sizeof(unsigned long long), s->stream);
   if (e == hipSuccess)
@@ -660,6 +713,8 @@ void pxg_stream_destroy(pxg_stream* s) {
     (void)hipHostFree(s->hostCounts);
   if (s->hostCA)
     (void)hipHostFree(s->hostCA);
+  if (s->stage)
+    (void)hipHostFree(s->stage);
   if (s->stream)
     (void)hipStreamDestroy(s->stream);
   delete s;
@@ -721,10 +776,11 @@ int pxg_set_graphs(pxg_stream* s, int on) {
 int pxg_fetch_counts(pxg_stream* s, uint32_t first, uint32_t count) {
   if (!s || first + count > s->nLoaded)
     return fail(PXG_ERR_ARG, "pxg_fetch_counts: bad range");
-  PXG_HIP(hipMemcpyAsync(s->hostCounts + first, s->pool.counts + first, count * sizeof(EventCounts),
-                         hipMemcpyDeviceToHost, s->stream));
-  PXG_HIP(hipMemcpyAsync(s->hostCA + first, s->ca.cnt + first, count * sizeof(CACounts), hipMemcpyDeviceToHost,
-                         s->stream));
+  if (count) {
+    launchCountsOut(s->pool.counts + first, s->hostCountsDev + first, s->ca.cnt + first, s->hostCADev + first, count,
+                    s->stream);
+    PXG_HIP(hipGetLastError());
+  }
   PXG_HIP(hipStreamSynchronize(s->stream));
   uint32_t st = 0;
   for (uint32_t e = first; e < first + count; ++e) {
@@ -806,12 +862,31 @@ static int plainEvent(pxg_stream* s, const uint32_t* words, const uint8_t* fedId
     return fail(PXG_ERR_ARG, "null input");
   pxg_raw_view v{words, fedIds, nWords};
   pxg_beamspot bs{};
-  int rc = pxg_load_events(s, 1, &v, &bs);
+  int rc = describeEvents(s, 1, &v, &bs, 1);
   if (rc)
     return rc;
+  if (!s->stage)
+    PXG_HIP(allocStage(s));
+  // Through the stream's staging buffer with one kernel, where a copy per array would stage
+  // the caller's memory as well.  The call before has waited for the stream, and so does
+  // this one, so the buffer is free here and the caller's arrays are on return.
+  const size_t fedOffset = alignUp(nWords, 4);  // in words
+  if (nWords) {
+    std::memcpy(s->stage, words, size_t(nWords) * 4);
+    std::memcpy(s->stage + fedOffset, fedIds, nWords / 2);
+  }
+  const uint32_t nWords4 = (nWords + 3) / 4, nFeds16 = (nWords / 2 + 15) / 16;
+  loadOneKernel<<<(nWords4 + nFeds16) / 256 + 1, 256, 0, s->stream>>>(
+      reinterpret_cast<const uint4*>(s->stageDev), reinterpret_cast<uint4*>(s->pool.words), nWords4,
+      reinterpret_cast<const uint4*>(s->stageDev + fedOffset), reinterpret_cast<uint4*>(s->pool.fedIds), nFeds16,
+      s->pool.events, s->hostEvents[0]);
+  PXG_HIP(hipGetLastError());
+  markLoaded(s, 1);
   rc = runStages(s, 0, 1, 1, upto);
-  if (rc)
+  if (rc) {
+    (void)hipStreamSynchronize(s->stream);
     return rc;
+  }
   return pxg_fetch_counts(s, 0, 1);
 }
 

@@ -36,6 +36,10 @@ namespace pxg {
     constexpr int kMaxDevices = 64;
     std::mutex g_scratchMutex;
     uint8_t* g_scratchPtr[kMaxDevices] = {};  // each device's address of `scratch`
+    // an event's counters come back through mapped pinned memory, a slot per device that, like
+    // the scratch array, lasts as long as the process
+    EventCounts* g_hostCounts[kMaxDevices] = {};
+    EventCounts* g_hostCountsDev[kMaxDevices] = {};
 
     __global__ void setEventKernel(EventDesc* dst, EventDesc v) { *dst = v; }
   }  // namespace
@@ -52,6 +56,12 @@ namespace pxg {
       const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
       if (e != hipSuccess || !ptr)
         return fail(PXG_ERR_HIP, "hipGetSymbolAddress(scratch) on device %d: %s", device, hipGetErrorString(e));
+      hipError_t h = hipHostMalloc(reinterpret_cast<void**>(&g_hostCounts[device]), sizeof(EventCounts),
+                                   hipHostMallocDefault);
+      if (h == hipSuccess)
+        h = hipHostGetDevicePointer(reinterpret_cast<void**>(&g_hostCountsDev[device]), g_hostCounts[device], 0);
+      if (h != hipSuccess)
+        return fail(PXG_ERR_HIP, "host memory for the counters of device %d: %s", device, hipGetErrorString(h));
       g_scratchPtr[device] = static_cast<uint8_t*>(ptr);
       return 0;
     }
@@ -80,9 +90,12 @@ extern "C" int pxg_raw_to_cluster_noalloc(pxg_context* ctx, void* hipStream, con
     return fail(PXG_ERR_ARG, "pxg_raw_to_cluster_noalloc: device %d is current, the context is on %d", dev,
                 ctx->device);
   uint8_t* base = nullptr;
-  {
+  EventCounts *hostCounts = nullptr, *hostCountsDev = nullptr;
+  if (dev < kMaxDevices) {
     std::lock_guard<std::mutex> lock(g_scratchMutex);
-    base = dev < kMaxDevices ? g_scratchPtr[dev] : nullptr;
+    base = g_scratchPtr[dev];
+    hostCounts = g_hostCounts[dev];
+    hostCountsDev = g_hostCountsDev[dev];
   }
   if (!base)
     return fail(PXG_ERR_ARG, "pxg_raw_to_cluster_noalloc: no scratch address for device %d (pxg_init not run)",
@@ -128,9 +141,10 @@ extern "C" int pxg_raw_to_cluster_noalloc(pxg_context* ctx, void* hipStream, con
   e = hipGetLastError();
   if (e != hipSuccess)
     return fail(PXG_ERR_HIP, "pxg_raw_to_cluster_noalloc: launch failed: %s", hipGetErrorString(e));
-  EventCounts cnt{};
-  PXG_HIP(hipMemcpyAsync(&cnt, p.counts, sizeof(EventCounts), hipMemcpyDeviceToHost, s));
+  launchCountsOut(p.counts, hostCountsDev, nullptr, nullptr, 1, s);
+  PXG_HIP(hipGetLastError());
   PXG_HIP(hipStreamSynchronize(s));
+  const EventCounts cnt = *hostCounts;
   d->nModules = cnt.nModules;
   d->nDigis = nWords;
   c->nClusters = cnt.nClusters;

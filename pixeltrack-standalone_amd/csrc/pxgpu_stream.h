@@ -32,6 +32,12 @@ struct pxg_stream {
   std::vector<void*> owned;
   pxg::EventDesc* hostEvents = nullptr;    // pinned
   pxg::EventCounts* hostCounts = nullptr;  // pinned
+  // the counters' device addresses: the kernel that ends a call writes them to the host
+  pxg::EventCounts* hostCountsDev = nullptr;
+  pxg::CACounts* hostCADev = nullptr;
+  // the per-event entry points' raw words and FED ids, in mapped pinned memory
+  uint32_t* stage = nullptr;
+  uint32_t* stageDev = nullptr;
   uint32_t nLoaded = 0;
   uint32_t wordCapacity = 0;
   // per resident event: the last stage run on it since it was loaded (0 none), so that
@@ -92,6 +98,9 @@ namespace pxg::detail {
                        GatherSrc* table, const GatherSrc* tableDev);
   // bytes of device memory a pool of maxEvents events and maxWords words takes
   size_t poolBytes(uint32_t maxEvents, uint32_t maxWords, const CACapacities& caps);
+  // writes n events' counters (ca may be null) to mapped host memory, on stream s
+  void launchCountsOut(const EventCounts* counts, EventCounts* hostCounts, const CACounts* ca, CACounts* hostCA,
+                       uint32_t n, hipStream_t s);
   // destroys the stream's captured stage sequences
   void dropGraphs(pxg_stream* s);
   // looks up the device's address of the no-alloc entry point's scratch array (once per
