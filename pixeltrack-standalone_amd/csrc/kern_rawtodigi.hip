@@ -28,6 +28,7 @@ namespace pxg {
 
     struct Digi {
       uint32_t row, col, adcRaw, moduleId, rawId;
+      uint32_t gainFirst, colBytes;  // the module's gain table (SlotInfo)
     };
 
     // 0: no digi; 1: digi; 2: error record
@@ -89,9 +90,10 @@ namespace pxg {
       }
       if (slot >= kCablingSize)
         return 0;
-      const uint32_t rawId = m.RawId[slot];
-      const uint32_t rocInDet = m.rocInDet[slot];
-      if (m.badRocs[slot] || c.modToUnp[slot])
+      const SlotInfo info = c.slots[slot];
+      const uint32_t rawId = info.rawId;
+      const uint32_t rocInDet = (info.moduleAndRoc >> 16) & 0x7fff;
+      if (info.moduleAndRoc >> 31)
         return 0;
       const bool barrel = ((rawId >> 25) & 7) == 1;
       uint32_t layer = 0;
@@ -144,7 +146,9 @@ namespace pxg {
       d.row = uint32_t(row);
       d.col = uint32_t(col);
       d.adcRaw = w & kAdcMask;
-      d.moduleId = m.moduleId[slot];
+      d.moduleId = info.moduleAndRoc & 0xffff;
+      d.gainFirst = info.gainFirst;
+      d.colBytes = info.colBytes;
       d.rawId = rawId;
       return 1;
     }
@@ -152,16 +156,14 @@ namespace pxg {
     // gain/pedestal calibration; returns false for dead or noisy columns.
     // The arithmetic is kept in the serial program's order with no FMA
     // contraction (the library is compiled with -ffp-contract=off).
-    __device__ __forceinline__ bool calibrate(const DevConditions& c, uint32_t id, uint32_t row, uint32_t col,
-                                              uint32_t adcRaw, uint16_t& adcOut) {
+    __device__ __forceinline__ bool calibrate(const DevConditions& c, const Digi& d, uint16_t& adcOut) {
       const SiPixelGainForHLTonGPU& g = *c.gain;
+      const uint32_t id = d.moduleId, row = d.row, col = d.col, adcRaw = d.adcRaw;
       if (id >= kMaxNumModules || row >= kRowsPerModule || col >= kColsPerModule)
         return false;  // outside the calibration tables (the reference reads out of bounds)
-      const GainRangeAndCols rc = g.rangeAndCols[id];
-      if (rc.nCols <= 0)
+      if (d.gainFirst == kNoGain)
         return false;
-      const uint32_t colBytes = (rc.second - rc.first) / uint32_t(rc.nCols);
-      const uint32_t offset = rc.first + col * colBytes + 2 * (row / g.numberOfRowsAveragedOver_);
+      const uint32_t offset = d.gainFirst + col * d.colBytes + 2 * (row / g.numberOfRowsAveragedOver_);
       if (offset + 2 > c.gainDataBytes)
         return false;
       const GainDecoding s = c.gainData[offset / 2];
@@ -186,7 +188,7 @@ namespace pxg {
       if (decodeWord(c, words[g], fedIds[g >> 1], d, e) != 1)
         return kInvId;
       uint16_t a;
-      if (d.moduleId == kInvId || !calibrate(c, d.moduleId, d.row, d.col, d.adcRaw, a))
+      if (d.moduleId == kInvId || !calibrate(c, d, a))
         return kInvId;
       return d.moduleId;
     }
@@ -194,7 +196,10 @@ namespace pxg {
   }  // namespace
 
   // a (blocks per event, events) grid, an event's blocks on one XCD: the event of a
-  // workgroup is its grid row, with no search over the events' block offsets
+  // workgroup is its grid row, with no search over the events' block offsets.  Bound: its
+  // chain of gathers (the slot's record, then the gain), so the record holds what eight
+  // tables did, and only a workgroup's first wave decodes words before its own: 128 PU50
+  // events 124 to 83 us.
   __global__ void __launch_bounds__(kDecodeBlock) decodeKernel(DevConditions c, Pool p) {
     const LogicalBlock lb = logicalBlock();
     const uint32_t e = lb.y;
@@ -226,7 +231,7 @@ namespace pxg {
         rawId = d.rawId;
         moduleInd = uint16_t(d.moduleId);
         if (moduleInd != kInvId) {
-          if (calibrate(c, d.moduleId, d.row, d.col, d.adcRaw, adc)) {
+          if (calibrate(c, d, adc)) {
             id = moduleInd;
           } else {
             moduleInd = kInvId;
@@ -251,12 +256,21 @@ namespace pxg {
     const uint64_t below = vmask & ((1ull << lane) - 1ull);
     const int prevLane = below ? 63 - __clzll(below) : -1;
     const uint32_t prevId = __shfl(id, prevLane < 0 ? 0 : prevLane);
-    // the first valid lane of the wave looks back across the wave start
+    // The first valid lane of the wave looks back across the wave start: at the last valid
+    // digis of the workgroup's earlier waves, and past the workgroup's first word by decoding
+    // the words before it.
+    __shared__ uint32_t sLast[kDecodeBlock / 64];
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t lastId = __shfl(id, vmask ? 63 - __clzll(vmask) : 0);
+    if (lane == 0)
+      sLast[wave] = vmask ? lastId : kInvId;
+    __syncthreads();
     uint32_t carry = kInvId;
     const uint32_t firstValid = vmask ? __ffsll((unsigned long long)vmask) - 1 : 64;
     if (lane == firstValid) {
-      const uint32_t waveStart = local - lane;  // local index of lane 0
-      for (uint32_t j = waveStart; j > 0; --j) {
+      for (uint32_t w = wave; w > 0 && carry == kInvId; --w)
+        carry = sLast[w - 1];
+      for (uint32_t j = carry == kInvId ? lb.x * kDecodeBlock : 0; j > 0; --j) {
         carry = validModuleAt(c, p.words, p.fedIds, wordOffset + j - 1);
         if (carry != kInvId)
           break;

@@ -579,12 +579,34 @@ int pxg_init(const pxg_conditions* c, pxg_context** out) {
     ctx->owned.push_back(dst);
     return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
   };
-  void *cab, *m2u, *gain, *gdata, *com, *det, *lay, *avg;
+  // the decoder's view of the cabling and gain tables
+  std::vector<SlotInfo> slots(kCablingSize);
+  {
+    const auto& m = *static_cast<const SiPixelFedCablingMapGPU*>(c->cabling);
+    const auto& g = *static_cast<const SiPixelGainForHLTonGPU*>(c->gain);
+    for (uint32_t i = 0; i < kCablingSize; ++i) {
+      SlotInfo& v = slots[i];
+      const uint32_t id = m.moduleId[i];
+      const bool skip = m.badRocs[i] || c->mod_to_unp[i];
+      v.rawId = m.RawId[i];
+      // an id that does not fit is no module; the decoder tells it from kInvId, "no id"
+      const uint32_t id16 = id <= 0xffff ? id : (id & 0xffff) == kInvId ? uint32_t(kInvId) : 0xffffu;
+      v.moduleAndRoc = id16 | std::min(m.rocInDet[i], 0x7fffu) << 16 | uint32_t(skip) << 31;
+      v.gainFirst = kNoGain;
+      v.colBytes = 0;
+      if (id < kMaxNumModules && g.rangeAndCols[id].nCols > 0) {
+        const GainRangeAndCols& r = g.rangeAndCols[id];
+        v.gainFirst = r.first;
+        v.colBytes = (r.second - r.first) / uint32_t(r.nCols);
+      }
+    }
+  }
+  void *cab, *slt, *gain, *gdata, *com, *det, *lay, *avg;
   hipError_t e = hipGetDevice(&ctx->device);
   if (e == hipSuccess)
     e = up(c->cabling, sizeof(SiPixelFedCablingMapGPU), cab);
   if (e == hipSuccess)
-    e = up(c->mod_to_unp, kCablingSize, m2u);
+    e = up(slots.data(), slots.size() * sizeof(SlotInfo), slt);
   if (e == hipSuccess)
     e = up(c->gain, sizeof(SiPixelGainForHLTonGPU), gain);
   if (e == hipSuccess)
@@ -601,7 +623,7 @@ int pxg_init(const pxg_conditions* c, pxg_context** out) {
     pxg_finalize(ctx);
     return fail(PXG_ERR_HIP, "pxg_init: %s", hipGetErrorString(e));
   }
-  ctx->cond = {static_cast<const SiPixelFedCablingMapGPU*>(cab), static_cast<const uint8_t*>(m2u),
+  ctx->cond = {static_cast<const SiPixelFedCablingMapGPU*>(cab), static_cast<const SlotInfo*>(slt),
                static_cast<const SiPixelGainForHLTonGPU*>(gain), static_cast<const GainDecoding*>(gdata),
                c->gain_data_bytes,
                static_cast<const CPECommonParams*>(com),      static_cast<const CPEDetParams*>(det),

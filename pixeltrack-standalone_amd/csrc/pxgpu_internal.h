@@ -38,10 +38,21 @@ namespace pxg {
     kStatusHitOverflow = 1u << 3,      // more than 48k clusters in the event
   };
 
+  // What the decoder needs of a cabling slot and of its module's gain table, gathered once
+  // when the conditions are uploaded: one 16-byte load per word where the tables are eight.
+  struct alignas(16) SlotInfo {
+    uint32_t rawId;
+    uint32_t moduleAndRoc;  // module id | ROC in module << 16 | slot not used (bad or to be skipped) << 31
+    uint32_t gainFirst;     // byte offset of the module's first gain column, or kNoGain
+    uint32_t colBytes;      // bytes of a gain column
+  };
+  static_assert(sizeof(SlotInfo) == 16, "one load");
+  constexpr uint32_t kNoGain = 0xffffffffu;
+
   // Conditions resident on the device, uploaded once (immutable afterwards).
   struct DevConditions {
     const SiPixelFedCablingMapGPU* cabling;
-    const uint8_t* modToUnp;
+    const SlotInfo* slots;  // [kCablingSize]
     const SiPixelGainForHLTonGPU* gain;  // v_pedestals unused: see gainData
     const GainDecoding* gainData;
     uint32_t gainDataBytes;
