@@ -1,5 +1,5 @@
-// Self-test entry point of the fast duplicate remover (csrc/kern_classify.hip) on track
-// lists the caller makes up, for tests/test_gpu_duplicates.py.  Test support only; the
+// Self-test entry points of the fast duplicate remover and the triplet cleaner
+// (csrc/kern_classify.hip) on lists the caller makes up, for tests/test_gpu_duplicates.py.  Test support only; the
 // reconstruction library does not load it.
 #include "../../pixeltrack-standalone_amd/csrc/kern_classify.hip"
 
@@ -35,5 +35,25 @@ extern "C" int pxs_fast_duplicates(uint32_t nTuples, uint32_t nCells, uint32_t n
   ca.dupOwner = dupOwner;
   dupActiveKernel<<<dim3(blocks, 1), kCaBlock>>>(ca);
   fastDuplicateKernel<<<1, kEventBlock>>>(ca);
+  return hipDeviceSynchronize() == hipSuccess && hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// One event of nHits hits with the tuples bins[hitOff[h]] to bins[hitOff[h + 1] - 1] in any
+// order, each of tupleOff[t + 1] - tupleOff[t] hits.  Device arrays; layerStart: sixteen
+// entries, the tenth nHits; state as above.
+extern "C" int pxs_triplet_cleaner(uint32_t nTuples, uint32_t nHits, uint32_t nBins, uint32_t* layerStart,
+                                   uint32_t* hitOff, uint32_t* bins, uint32_t* tupleOff, uint8_t* quality,
+                                   float* state, uint32_t blocks) {
+  using namespace pxg;
+  Pool p{};
+  p.hitsLayerStart = layerStart;
+  CAPool ca{};
+  ca.caps = {64, nTuples, nTuples, nBins, 64, 128};
+  ca.tupleOff = tupleOff;
+  ca.h2tOff = hitOff;
+  ca.h2tBins = bins;
+  ca.quality = quality;
+  ca.state = state;
+  tripletCleanerKernel<<<dim3(blocks, 1), kCaBlock>>>(p, ca);
   return hipDeviceSynchronize() == hipSuccess && hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -1,9 +1,13 @@
-"""The fast duplicate remover's rounds (csrc/kern_classify.hip) on made-up track lists
-against the serial loop (CAHitNtupletGeneratorKernelsImpl.h:151-189): cells in ascending
+"""The duplicate removers (csrc/kern_classify.hip) on made-up lists.
+
+The fast duplicate remover's rounds against the serial loop (CAHitNtupletGeneratorKernelsImpl.h:151-189): cells in ascending
 order, each keeping its loose tuple of smallest |tip|.  The lists reach what events seldom
 do: more loose tuples in a cell than the kernel keeps beside it, more tuples than the
 slot table has entries, long chains of cells that each wait for the one before, more cells
-than threads, tied impact parameters."""
+than threads, tied impact parameters.
+
+The triplet cleaner against the serial loop over hits (:479-534), with lists around what a
+wavefront stages in LDS for its 64 hits."""
 import ctypes as C
 import os
 
@@ -75,3 +79,50 @@ def test_rounds_match_the_serial_loop(n_tuples, n_cells, width, loose):
     assert lib.pxs_fast_duplicates(stride, space, n_cells, *[x.data_ptr() for x in t], 8) == 0
     got = t[4].cpu().numpy()[:n_tuples]
     assert np.array_equal(got, want), f"{(got != want).sum()} of {n_tuples} qualities differ"
+
+
+@pytest.mark.parametrize("lengths", [
+    [0, 0, 1, 0],
+    [3] * 64 + [5] * 7,        # a full wavefront and a ragged one
+    [16] * 64,                 # exactly what is staged
+    [16] * 63 + [17],          # one entry more: worked in memory
+    [0] * 10 + [900] + [2] * 53 + [40] * 64 + [1, 2],
+])
+def test_triplet_cleaner_matches_the_serial_loop(lengths):
+    import torch
+    lib = C.CDLL(LIB)
+    vp, u32 = C.c_void_p, C.c_uint32
+    lib.pxs_triplet_cleaner.argtypes = [u32, u32, u32] + [vp] * 6 + [u32]
+    rng = np.random.default_rng(len(lengths))
+    n = 2048
+    size = rng.choice([3, 3, 3, 4, 5], n)
+    size[rng.random(n) < 0.3] = 3
+    tip = rng.choice(np.linspace(-0.4, 0.4, 57), n).astype(np.float32)  # ties among them
+    off = np.concatenate([[0], np.cumsum(size)]).astype(np.int32)
+    lists = [rng.choice(np.nonzero(size == 3)[0] if rng.random() < 0.5 else n, m, replace=False) for m in lengths]
+    want = np.full(n, LOOSE, np.uint8)
+    order = [np.sort(l)[::-1] for l in lists]
+    for l in order:
+        if len(l) < 2:
+            continue
+        most = size[l].max()
+        want[l[size[l] != most]] = DUP
+        if most == 3:
+            score = np.abs(tip[l])
+            want[np.delete(l, np.argmin(score))] = DUP
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+    hoff = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    flat = np.concatenate(lists).astype(np.int32) if hoff[-1] else np.zeros(1, np.int32)
+    layers = np.zeros(16, np.int32)
+    layers[10] = len(lengths)
+    state = np.zeros((5, n), np.float32)
+    state[1] = tip
+    t = [dev(layers), dev(hoff), dev(flat), dev(off), dev(np.full(n, LOOSE, np.uint8)), dev(state)]
+    torch.cuda.synchronize()
+    assert lib.pxs_triplet_cleaner(n, len(lengths), len(flat), *[x.data_ptr() for x in t], 3) == 0
+    if hoff[-1]:
+        assert np.array_equal(t[2].cpu().numpy(), np.concatenate(order)), "order within the lists"
+    assert np.array_equal(t[4].cpu().numpy(), want)
