@@ -1137,9 +1137,11 @@ namespace pxg {
     // rank in the workgroup (high 14 bits) plus its tuples placed so far (low 18 bits; a
     // cell has fewer than 2^18 tuples), so the second pass reads no slot from memory.
     // Slot s records its cell and the cell's tuple count (the walk's scratch is free now),
-    // so the later passes visit only the cells that are in tuples.  Workgroup 0 of each
+    // so the later passes visit only the cells that are in tuples; the cells in two or more
+    // are listed beside, in the same order, with their slots.  Workgroup 0 of each
     // event also finalises the tuple offsets (HistoContainer.h:193-204 bulkFinalizeFill).
     constexpr uint32_t kTrSlice = 16384;       // cells per slice: 64 KB of counts
+    constexpr uint32_t kNoList = 0xffffffffu;
     constexpr uint32_t kTrGroupCells = 40960;  // capacity cells per workgroup: 12 per event at
                                                // 458752 cells, one slice each up to 196608 cells
     static_assert(kTrSlice <= (1u << 14) && kCapsReference.maxTuples < (1u << 18) &&
@@ -1150,7 +1152,7 @@ namespace pxg {
       const uint32_t s = blockIdx.x, e = blockIdx.y;
       __shared__ uint32_t cnt[kTrSlice];
       __shared__ uint32_t lds[kEventBlock / 64];
-      __shared__ uint32_t sBase;
+      __shared__ uint32_t sBase, sMulti;
       const CACounts cn = ca.cnt[e];
       const size_t cb = ca.cellBase(e);
       const size_t tb = ca.tupleBase(e);
@@ -1187,6 +1189,7 @@ namespace pxg {
       const uint4* cells4 = reinterpret_cast<const uint4*>(ca.tupleCells + 4 * tb);
       uint32_t* trCells = ca.dfsT + cb;
       uint32_t* trTotal = ca.dfsH + cb;
+      uint32_t* multiSlots = ca.startCells + cb;
       TupleIndex* pool = ca.trPool + size_t(e) * ca.caps.maxCellLists * kCaMaxCellTracks;
       uint32_t status = 0;
       for (uint32_t c0 = s * kTrSlice; c0 < cn.nCells; c0 += gridDim.x * kTrSlice) {
@@ -1215,36 +1218,57 @@ namespace pxg {
         };
         forSlice([&](uint32_t i, uint32_t) { atomicAdd(&cnt[i], 1u); });
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < n; i += kEventBlock)
-          if (cnt[i] == 0) {
-            ca.trSlot[cb + c0 + i] = -1;
-            ca.trCount[cb + c0 + i] = 0;
-          }
-        const uint32_t per = (n + kEventBlock - 1) / kEventBlock;
-        const uint32_t i0 = min(threadIdx.x * per, n), i1 = min(i0 + per, n);
-        uint32_t mine = 0;
-        for (uint32_t i = i0; i < i1; ++i)
-          mine += cnt[i] > 0;
-        uint32_t total;
-        uint32_t rank = wgExclusiveScan<kEventBlock>(mine, total, lds);
-        if (threadIdx.x == 0)
-          sBase = total ? atomicAdd(&ca.cnt[e].trLists, total) : 0;
+        // slots in cell order: each wavefront takes consecutive cells, 64 at a time, so that
+        // their counts and the stores of their slots are coalesced (with consecutive cells per
+        // thread 12 PU200 events took 388 us, so 323)
+        constexpr uint32_t kWaves = kEventBlock / 64, kPerWave = kTrSlice / kWaves;
+        static_assert(kPerWave % 64 == 0, "whole wavefronts");
+        const uint32_t lane = laneId(), wave = threadIdx.x >> 6, first = wave * kPerWave;
+        auto countOf = [&](uint32_t i) { return i < n ? cnt[i] : 0; };
+        uint32_t mine = 0;  // cells with tuples, and above them those with two or more
+        for (uint32_t r = 0; r < kPerWave; r += 64) {
+          const uint32_t k = countOf(first + r + lane);
+          mine += uint32_t(__popcll(__ballot(k > 0))) + (uint32_t(__popcll(__ballot(k > 1))) << 16);
+        }
+        if (lane == 0)
+          lds[wave] = mine;
         __syncthreads();
-        for (uint32_t i = i0; i < i1; ++i) {
-          const uint32_t k = cnt[i];
-          if (k == 0)
-            continue;
-          const uint32_t slot = sBase + rank++;
-          const uint32_t c = c0 + i;
-          if (slot + 1 < ca.caps.maxCellLists) {
-            ca.trSlot[cb + c] = int32_t(slot);
-            trCells[slot] = c;
-            trTotal[slot] = k;
-          } else {
-            ca.trSlot[cb + c] = -2;
-            status |= kCaTrackStoreOverflow;
+        uint32_t before = 0, total = 0;
+        for (uint32_t w = 0; w < kWaves; ++w) {
+          before += w < wave ? lds[w] : 0;
+          total += lds[w];
+        }
+        if (threadIdx.x == 0)
+          sBase = total & 0xffffu ? atomicAdd(&ca.cnt[e].trLists, total & 0xffffu) : 0;
+        if (threadIdx.x == 64)
+          sMulti = total >> 16 ? atomicAdd(&ca.cnt[e].nMulti, total >> 16) : 0;
+        __syncthreads();
+        uint32_t rank = before & 0xffffu, multi = before >> 16;
+        for (uint32_t r = 0; r < kPerWave; r += 64) {
+          const uint32_t i = first + r + lane, k = countOf(i), c = c0 + i;
+          const uint64_t some = __ballot(k > 0), several = __ballot(k > 1);
+          const uint32_t at = rank + __popcll(some & lanesBelow()), slot = sBase + at;
+          const bool stored = slot + 1 < ca.caps.maxCellLists;
+          if (i < n) {
+            ca.trSlot[cb + c] = k == 0 ? -1 : stored ? int32_t(slot) : -2;
+            ca.trCount[cb + c] = uint16_t(stored ? min(k, kCaMaxCellTracks) : 0u);
           }
-          cnt[i] = (rank - 1) << 18;  // the list's rank in the workgroup above, tuples placed below
+          if (k > 0) {
+            if (stored) {
+              trCells[slot] = c;
+              trTotal[slot] = k;
+            } else {
+              status |= kCaTrackStoreOverflow;
+            }
+            cnt[i] = at << 18;  // the list's rank in the workgroup above, tuples placed below
+          }
+          if (k > 1) {
+            const uint32_t m = sMulti + multi + __popcll(several & lanesBelow());
+            ca.multiCells[cb + m] = c;
+            multiSlots[m] = stored ? slot : kNoList;  // no list: nothing to sort or to clean
+          }
+          rank += __popcll(some);
+          multi += __popcll(several);
         }
         __syncthreads();
         forSlice([&](uint32_t i, uint32_t t) {
@@ -1258,27 +1282,33 @@ namespace pxg {
         atomicOr(&ca.cnt[e].status, status);
     }
 
-    // sorts each cell's track list (ascending tuple index, first 48 kept) and
-    // runs a16 kernel_earlyDuplicateRemover (CAHitNtupletGeneratorKernelsImpl.h:126-149)
-    // on it: order independent, it only marks shorter tuples as duplicates.
+    // Sorts the track list of each cell in two or more tuples (ascending tuple index, first
+    // 48 kept) and runs a16 kernel_earlyDuplicateRemover (CAHitNtupletGeneratorKernelsImpl.h:
+    // 126-149) on it: order independent, it only marks shorter tuples as duplicates.
+    // Bound: the cache lines of the lists and of their tuples' offsets.  The lists of one
+    // tuple (three in five at PU50) are not visited: 128 PU50 events 104 to 93 us, 12 PU200
+    // events 106 to 73, one PU200 event 44 to 25.
     __global__ void __launch_bounds__(kCaBlock) trackListSortKernel(CAPool ca) {
       const uint32_t e = logicalBlock().y;
-      const uint32_t nT = ca.cnt[e].nTuples;
+      const uint32_t nT = ca.cnt[e].nTuples, nMulti = ca.cnt[e].nMulti;
       const size_t cb = ca.cellBase(e);
       const size_t tb = ca.tupleBase(e);
       TupleIndex* pool = ca.trPool + size_t(e) * ca.caps.maxCellLists * kCaMaxCellTracks;
       const uint32_t* off = ca.tupleOff + ca.offBase(e);
-      const uint32_t* trCells = ca.dfsT + cb;
       const uint32_t* trTotal = ca.dfsH + cb;
-      const uint32_t nLists = min(ca.cnt[e].trLists, ca.caps.maxCellLists - 1);
+      const uint32_t* multiSlots = ca.startCells + cb;
       uint32_t status = 0;
-      for (uint32_t slot = gridStart(); slot < nLists; slot += gridStride()) {
-        const uint32_t c = trCells[slot], total = trTotal[slot];
+      for (uint32_t i = gridStart(); i < nMulti; i += gridStride()) {
+        const uint32_t slot = multiSlots[i];
+        if (slot == kNoList)
+          continue;
+        const uint32_t total = trTotal[slot];
         TupleIndex* list = pool + size_t(slot) * kCaMaxCellTracks;
         uint32_t n = total;
         if (total > kCaMaxCellTracks) {
           // keep the 48 smallest tuple indices: rebuild from the tuples
           status |= kCaTrackOverflow;
+          const uint32_t c = ca.multiCells[cb + i];
           n = 0;
           for (uint32_t t = 0; t < nT && n < kCaMaxCellTracks; ++t)
             for (int k = 0; k < 4; ++k) {
@@ -1301,17 +1331,12 @@ namespace pxg {
             list[m] = v;
           }
         }
-        ca.trCount[cb + c] = uint16_t(n);
-        if (n < 2)
-          continue;
         uint32_t maxNh = 0;
         for (uint32_t k = 0; k < n; ++k)
           maxNh = max(maxNh, off[list[k] + 1] - off[list[k]]);
         for (uint32_t k = 0; k < n; ++k)
           if (off[list[k] + 1] - off[list[k]] != maxNh)
             ca.quality[tb + list[k]] = kQualityDup;
-        const uint32_t at = waveAlloc(&ca.cnt[e].nMulti, true);
-        ca.multiCells[cb + at] = c;
       }
       if (status)
         atomicOr(&ca.cnt[e].status, status);

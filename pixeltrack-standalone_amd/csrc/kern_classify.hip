@@ -112,8 +112,8 @@ namespace pxg {
         uint32_t keep[kDupLooseCap];
         if (k < nMulti) {
           c = multi[k];
-          const TupleIndex* list = pool + size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks;
-          const uint32_t n = ca.trCount[cb + c];
+          const uint32_t n = ca.trCount[cb + c];  // 0: the store had no list for it
+          const TupleIndex* list = pool + (n ? size_t(ca.trSlot[cb + c]) * kCaMaxCellTracks : 0);
           for (uint32_t a = 0; a < n; ++a) {
             const TupleIndex it = list[a];
             if (q[it] != kQualityLoose)
