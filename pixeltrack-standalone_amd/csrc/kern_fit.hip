@@ -5,11 +5,11 @@
 // The small symmetric positive-definite systems ((N + 1) x (N + 1) at most)
 // are solved through an LDL^T factorisation held in registers.
 //
-// Triplets and quadruplets run as two kernels, each with its own register
-// footprint, and the double-precision atan2, sin, cos and log are called, not
-// inlined: inlined, the unrolled loops interleaved N of them at once and the
-// fit needed about 370 registers per lane (one wave per SIMD).  Called, the
-// triplet fit takes 146 and the quadruplet fit 168 (three waves per SIMD).
+// Triplets and quadruplets share a launch, a size per workgroup and step, and the
+// double-precision atan2, sin, cos and log are called, not inlined: inlined,
+// the unrolled loops interleaved N of them at once and the fit needed about
+// 370 registers per lane (one wave per SIMD).  Called, it takes 168 (three
+// waves per SIMD).
 #include <hip/hip_runtime.h>
 
 #include "pxgpu_internal.h"
@@ -508,22 +508,36 @@ namespace pxg {
       ca.chi2[tb + tkid] = float((Ci.chi2 + L.chi2) / (2 * N - 5));
     }
 
-    // the fits of the tuples with N hits: sizes 3, then 4 and 5 (fitted on 4 hits)
-    template <int N>
+    // The fits of the tuples with 4 and 5 hits (on 4 of them), then of those with 3, in one
+    // launch: 256 entries of one size per workgroup and step.  A fit is a chain of dependent
+    // double-precision operations, so when few tuples leave the device idle both sizes side
+    // by side take what the longer takes, and for many the last waves of one size no longer
+    // run alone: against a launch per size, one PU50 event 33 to 22 us, 16 events 52 to 35,
+    // 128 events 160 to 143, 12 PU200 events 184 to 181.
     __global__ void __launch_bounds__(256, 3) fitKernel(DevConditions cond, Pool p, CAPool ca, double B) {
-      const uint32_t e = logicalBlock().y;
+      const LogicalBlock lb = logicalBlock();
+      const uint32_t e = lb.y;
       const uint32_t* mo = ca.multOff + size_t(e) * 16;
       const TupleIndex* mb = ca.multBins + size_t(e) * ca.caps.maxTuplesMult;
-      const uint32_t begin = N == 3 ? mo[3] : mo[4], end = N == 3 ? mo[4] : mo[6];
-      for (uint32_t k = begin + logicalBlock().x * blockDim.x + threadIdx.x; k < end; k += gridDim.x * blockDim.x)
-        fitTuple<N>(cond, p, ca, e, mb[k], B);
+      const uint32_t b3 = mo[3], b4 = mo[4], end = mo[6];
+      const uint32_t n4 = (end - b4 + 255) / 256, n3 = (b4 - b3 + 255) / 256;
+      for (uint32_t step = lb.x; step < n4 + n3; step += gridDim.x) {  // uniform per workgroup
+        if (step < n4) {
+          const uint32_t k = b4 + step * 256 + threadIdx.x;
+          if (k < end)
+            fitTuple<4>(cond, p, ca, e, mb[k], B);
+        } else {
+          const uint32_t k = b3 + (step - n4) * 256 + threadIdx.x;
+          if (k < b4)
+            fitTuple<3>(cond, p, ca, e, mb[k], B);
+        }
+      }
     }
   }  // namespace
 
   void launchFit(const CALaunch& l) {
     l.t->b("fit");
-    fitKernel<3><<<dim3(l.blocks, l.nEvents), 256, 0, l.s>>>(*l.cond, *l.p, *l.ca, l.bField);
-    fitKernel<4><<<dim3(l.blocks, l.nEvents), 256, 0, l.s>>>(*l.cond, *l.p, *l.ca, l.bField);
+    fitKernel<<<dim3(l.blocks, l.nEvents), 256, 0, l.s>>>(*l.cond, *l.p, *l.ca, l.bField);
     l.t->e();
   }
 
